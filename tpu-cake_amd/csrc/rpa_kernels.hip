@@ -2006,41 +2006,58 @@ __device__ __forceinline__ void pf_role(const Params& p, const SeqInfo wsi[4], i
 // ---------------------------------------------------------------------------------------------
 // prefill tiles of the co-resident layout (Params::co): 4-wave workgroups, 128-row tiles
 // ---------------------------------------------------------------------------------------------
-// A tile is (sequence, kv head, 128 / G tokens); wave w owns rows 32w .. 32w+31 as two 16-row MFMA
-// blocks, its queries in registers.  K/V chunks (32 keys) go from HBM straight into LDS with
-// gfx950's global_load_lds_dwordx4 (no registers held for data in flight), into a ring of four
-// 16 KiB slots, three chunks ahead of the compute.  Slot layout: K as 256-byte key rows whose
-// 16-byte column groups sit at group ^ (key % 16) (conflict-free A fragment reads), then V as
-// 256-byte key rows whose 32-byte dim blocks sit at block ^ (key % 8) (conflict-free transposing
-// reads, read_vt_fragments_x).  Each DMA instruction writes one contiguous KiB (64 lanes x 16 B);
-// the lane's source address picks which piece lands where.  The chunks' page ids come from a
-// table the workgroup copies into LDS per segment of up to kCoPages pages.
+// A tile is (sequence, kv head, 128 / G tokens); wave w owns rows 32w .. 32w+31 as one 32-row MFMA
+// block (v_mfma_f32_32x32x16_bf16), its queries in registers.  Operand layouts of that instruction:
+// A[i][k] and B[k][j] place row i / column j at lane % 32 and k = 8 (lane / 32) + e (e = element
+// 0..7); D[i][j] sits at lane % 32 = j, element v <-> i = 8 (v / 4) + 4 (lane / 32) + v % 4.  So
+//   S^T = K Q^T   A = K [32 keys x 16 dims], B = Q^T: a lane holds 16 of a chunk's 32 scores of ONE
+//                 query row (its other 16 are in lane ^ 32): a row maximum is 15 VALU maxima and one
+//                 v_permlane32_swap
+//   O^T += V^T P^T  A = V^T [32 dims x 16 keys], B = P^T [16 keys x 32 rows], key of slot e of
+//                 16-key step t: 16t + 8 (e / 4) + 4 (lane / 32) + e % 4 -- the keys the lane already
+//                 holds (elements 8t .. 8t+7 of S), so P needs no cross-lane movement.
+//
+// The step is software-pipelined over chunks: step c computes S of chunk c + 1 and adds P V of chunk
+// c - 1 (MFMA) while it takes the softmax of chunk c (VALU): no result of a step's MFMAs is used by
+// the same step, so a wave's VALU work fills the issue slots its MFMAs leave.  (A 32x32x16 MFMA
+// occupies the matrix cores for 32 cycles and the issue port for 4; up to six FMAs, or three and an
+// exponential, between two of them are free in a bare loop.)
+//
+// What bounds a step is the issue of its ~155 instructions per wave (a wave issues one in ~5 cycles
+// here) beside 512 matrix-core cycles, so the loop is unrolled over the four ring slots (addresses
+// become immediates) and each MFMA is followed by its share of the softmax.  Four prompts of 2048-6144
+// tokens, Hq 32 / Hkv 8, page 64: 425 -> 384 us per call (0.85 -> 0.94 PFLOP/s) against the 16x16x32 form
+// with QK^T, softmax and PV in sequence; 24 decode rows beside four 512-token chunks: 136 -> 124 us.
+//
+// K/V chunks (32 keys) go from HBM straight into LDS with gfx950's global_load_lds_dwordx4 (no
+// registers held for data in flight) into a ring of four K slots (chunks c + 1 .. c + 4 at step c) and
+// one of four V slots (c - 1 .. c + 2).  Each DMA instruction writes one contiguous KiB (64 lanes x
+// 16 B): kBlkKeys key rows of 2 DT bytes.  K: the 16-byte dim group g of a key sits at g ^ xk(key) and
+// blocks are kKPad bytes apart further than their KiB, so that the 16 keys of a 16-lane group of one
+// A fragment read fall on all 64 banks; V: the 64-byte dim group sits at g ^ xv(key), so that the four
+// keys of a transposing read's 32 lanes do.  The lane's source address picks which piece lands where.
+// The chunks' places come from a table the workgroup makes in LDS per segment: each chunk's address
+// (page size a multiple of 32: a chunk lies in one page), else each key's pool row.
 //
 // Waits: the DMA is issued from inline asm, so the compiler neither sees nor counts it, and the
-// only loads in the step loop are those DMAs (kCoDmas per wave per chunk).  The step's barrier
-// (co_barrier) therefore waits with an exact vmcnt for this wave's share of the chunk it is about
-// to read, and the barrier makes every wave's share visible.  (Issued as the compiler's builtin,
-// the DMA makes it wait for every DMA in flight before each LDS read it cannot tell apart,
-// draining the ring every step.)  No load in asm writes a register: a register the compiler
-// believed loaded could be reused before the load lands.
+// only loads in the step loop are those DMAs.  The step's barrier (co_barrier) therefore waits with an
+// exact vmcnt for this wave's share of the chunks it is about to read, and the barrier makes every
+// wave's share visible.  (Issued as the compiler's builtin, the DMA makes it wait for every DMA in
+// flight before each LDS read it cannot tell apart, draining the ring every step.)  No load in asm
+// writes a register: a register the compiler believed loaded could be reused before the load lands.
 //
 // Scaled bf16 and fp8 pools (the reference dequantises K and V as bf16(float(x) * scale),
-// ragged_paged_attention.py:124-129) add one pass per chunk, one step ahead of its compute, so the
-// step keeps one barrier: scaled bf16 chunks are scaled in place in their ring slot; fp8 chunks
-// (half the bytes) land in a ring of four 8 KiB code slots and are converted into a double buffer
-// of bf16 slots of the layout above, with the page's K and V scales (per (page, kv head), from a
-// table loaded with the page ids).
+// ragged_paged_attention.py:124-129) add one pass per step, over K of chunk c + 2 and V of chunk c:
+// scaled bf16 in place in their ring slots; fp8 chunks (half the bytes) land in rings of four code
+// slots and are converted into double-buffered bf16 slots of the layouts above.  fp8 K of a chunk in
+// one page converts exactly and the page's K scale multiplies the fp32 scores.
 constexpr int kCoWaves = 4;
-constexpr int kCoSlot = 16384;                    // one chunk: K (8 KiB) + V (8 KiB)
-constexpr int kCoSlots = 4;
-constexpr int kCoCodeSlot = 8192;                 // one fp8 chunk: K codes (4 KiB) + V codes (4 KiB)
-constexpr int kCoOrderBase = kCoSlots * kCoSlot;  // tile order tables (2 x kPfOrderMax ints)
-constexpr int kCoPages = 128;                     // page-id table entries (and fp8 scale pairs)
-constexpr int kCoPageBase = kCoOrderBase + 2 * kPfOrderMax * 4;
-constexpr int kCoScaleBase = kCoPageBase + kCoPages * 4;
-static_assert(kCoScaleBase + kCoPages * 8 <= kCoWaves * kWaveLds,
-              "co-resident prefill LDS exceeds the workgroup's allocation");
-static_assert(kCoSlots * kCoCodeSlot + 2 * kCoSlot <= kCoOrderBase, "fp8 code ring and bf16 buffers");
+
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ f32x16 mfma32(bf16x8 a, bf16x8 b, f32x16 c) {
+  return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0);
+}
 
 // Modes with co-resident prefill tiles.
 template <int MODE>
@@ -2048,21 +2065,55 @@ constexpr bool co_tiles() {
   return MODE == KV_BF16 || MODE == KV_BF16_SCALED || MODE == KV_FP8;
 }
 template <int MODE>
-constexpr int co_dmas() {  // DMA instructions per wave and chunk
-  return MODE == KV_FP8 ? 2 : 4;
-}
-template <int MODE>
-constexpr bool co_converts() {  // a pass per chunk one step ahead (scaled or fp8)
+constexpr bool co_converts() {  // a pass per step (scaled or fp8)
   return MODE != KV_BF16;
 }
 
-// The step's barrier: this wave's DMAs of the chunk the step reads first (chunk c, or c + 1 for the
-// modes that convert one step ahead) have landed -- N younger DMAs may still be in flight -- and
-// its LDS reads are done, then s_barrier.  A workgroup-scope release fence (__syncthreads) would
-// wait for every DMA in flight.
+// LDS geometry of a chunk of DT-wide key rows (DT 64, 128 or 256; narrower heads are padded to one).
+template <int DT>
+struct CoGeo {
+  static constexpr int kRow = 2 * DT;              // bytes of a key row
+  static constexpr int kBlkKeys = 1024 / kRow;     // keys per KiB block (one DMA)
+  static constexpr int kBlks = KV_CHUNK / kBlkKeys;
+  static constexpr int kKPad = DT == 256 ? 32 : 64, kVPad = DT == 256 ? 128 : 0;
+  static constexpr int kKBlk = 1024 + kKPad, kVBlk = 1024 + kVPad;
+  static constexpr int kKSlot = kBlks * kKBlk, kVSlot = kBlks * kVBlk;
+  static constexpr int kSteps = DT / 16;           // QK^T k-steps of 16 dims
+  static constexpr int kDb = DT / 32;              // PV dim blocks of 32
+  static __device__ __forceinline__ int xk(int key) { return DT == 64 ? (key >> 1) & 3 : DT == 128 ? key & 3 : key & 1; }
+  static __device__ __forceinline__ int xv(int key) { return DT == 64 ? (key >> 1) & 1 : DT == 128 ? key & 3 : key & 1; }
+};
+
+template <int MODE, int DT, bool UPG>
+struct CoLds {
+  using Geo = CoGeo<DT>;
+  static constexpr bool kFp8 = MODE == KV_FP8;
+  static constexpr int kCode = KV_CHUNK * DT;             // codes of one operand of a chunk
+  static constexpr int kCodeV = 4 * kCode;                // K codes at 0
+  static constexpr int kSlots = kFp8 ? 2 : 4;             // bf16 slots of V and of K
+  static constexpr int kV = kFp8 ? 8 * kCode : 0;
+  static constexpr int kK = kV + kSlots * Geo::kVSlot;
+  static constexpr int kOrder = kK + kSlots * Geo::kKSlot;  // tile order tables (2 x kPfOrderMax ints)
+  static constexpr int kSeqs = kOrder + 2 * kPfOrderMax * 4;  // the sequences' metadata (CoSeqs)
+  static constexpr int kTable = kSeqs + 4 * 256 * 4;
+  // a segment's table: its chunks' addresses (UPG), or its keys' pool rows; then (fp8) the scale pairs
+  static constexpr int kSegChunks = UPG ? 256 : kFp8 ? 16 : 32;
+  static constexpr int kEntries = UPG ? kSegChunks : kSegChunks * KV_CHUNK;
+  static constexpr int kScale = kTable + kEntries * (UPG ? 8 : 4);
+  static constexpr int kFlags = kScale + (kFp8 ? kEntries * 8 : 0);
+  static constexpr int kBytes = kFlags + kCoWaves * 4;
+  // DMAs per wave and step: kPerOp per operand; with fp8 rows of 64 bytes a wave carries one operand
+  static constexpr bool kOneOp = kFp8 && DT == 64;
+  static constexpr int kPerOp = kFp8 ? (DT >= 128 ? DT / 128 : 1) : Geo::kBlks / kCoWaves;
+  static constexpr int kStepDmas = kOneOp ? 1 : 2 * kPerOp;
+};
+
+// The step's barrier: all but the last N of this wave's DMAs have landed and its LDS reads and writes
+// are done, then s_barrier.  A workgroup-scope release fence (__syncthreads) would wait for every DMA
+// in flight.
 template <int N>
 __device__ __forceinline__ void co_barrier() {
-  static_assert(N >= 0 && N < 16, "co_barrier's vmcnt");
+  static_assert(N >= 0 && N < 64, "co_barrier's vmcnt");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
 
@@ -2074,269 +2125,558 @@ __device__ __forceinline__ uint32_t lds_addr_of(const void* ptr) {
   return (uint32_t)(uintptr_t)(const __attribute__((address_space(3))) void*)ptr;
 }
 
-// One 16-byte-per-lane DMA into the 1 KiB of LDS at lds_addr (wave-uniform); m0 is saved and
-// restored around it, so the compiler's use of m0 is untouched.
-__device__ __forceinline__ void co_dma(const void* src, uint32_t lds_addr) {
-  uint32_t save;
+// One 16-byte-per-lane DMA into the 1 KiB of LDS at lds_addr + imm (wave-uniform).
+__device__ __forceinline__ void co_dma(const void* src, uint32_t lds_addr, int imm) {
   asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %2\n\t"
+      "s_add_u32 m0, %1, %2\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, off\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(save)
-      : "v"(src), "s"(lds_addr)
-      : "memory");
+      "global_load_lds_dwordx4 %0, off"
+      :
+      : "v"(src), "s"(uni((int)lds_addr)), "i"(imm)
+      : "memory", "m0", "scc");
 }
 
 // The same DMA with the address split into a wave-uniform base (SGPRs) and a per-lane 32-bit byte
-// offset: the form for chunks whose every key exists, whose per-lane offsets are fixed for a tile.
-__device__ __forceinline__ void co_dma_s(const void* base, uint32_t off, uint32_t lds_addr) {
-  uint32_t save;
+// offset, which for a chunk's DMAs is fixed for a tile.
+__device__ __forceinline__ void co_dma_s(const void* base, uint32_t off, uint32_t lds_addr, int imm) {
   asm volatile(
-      "s_mov_b32 %0, m0\n\t"
-      "s_mov_b32 m0, %3\n\t"
+      "s_add_u32 m0, %2, %3\n\t"
       "s_nop 0\n\t"
-      "global_load_lds_dwordx4 %1, %2\n\t"
-      "s_mov_b32 m0, %0"
-      : "=&s"(save)
-      : "v"(off), "s"(base), "s"(lds_addr)
-      : "memory");
+      "global_load_lds_dwordx4 %0, %1"
+      :
+      : "v"(off), "s"(base), "s"(uni((int)lds_addr)), "i"(imm)
+      : "memory", "m0", "scc");
 }
 
-// Per-lane parts of the DMA addresses, the same for every chunk.  bf16: lane l of wave wv carries,
-// for t = 0, 1, key 4i + l/16 of block i = wv + 4t, and 16-byte LDS position l % 16 of that key's K
-// row (column group pos ^ (key % 16)) and V row (dims of 32-byte block (pos/2) ^ (key % 8), half
-// pos % 2).  fp8 (key[0], colk[0]): key 8 wv + l/8, bytes 16 (l % 8) .. +15 of its 128-byte row.
-struct CoLane {
-  int key[2];   // key within the chunk
-  int colk[2];  // element offset of the K piece within the key's row of kv head h
-  int colv[2];  // element offset of the V piece
-  uint32_t off[4];  // byte offsets from the chunk's first key row of kv head h: K pieces t = 0, 1, then V
+// A workgroup's chunk loads, the same for every tile: DMA t of this wave carries key key(t) of the
+// chunk, bytes colk(t) of its K row and colv(t) of its V row (from the first byte of the key's K row).
+// A narrow row's pieces wholly past D read the row's first piece (zero query dims, unstored outputs).
+template <int MODE, int DT, bool UPG>
+struct CoLoads {
+  using L = CoLds<MODE, DT, UPG>;
+  using Geo = CoGeo<DT>;
+  int wv, lane;
+  uint32_t row;              // bytes between consecutive keys of a page
+  int D;
+  uint32_t offk[L::kPerOp], offv[L::kPerOp];  // key(t) * row + colk(t) / colv(t)
+  uint32_t offt[L::kPerOp];                   // offv with keys past the current tile's last one read as it
+
+  __device__ __forceinline__ int blk(int t) const { return L::kOneOp ? wv & 1 : wv + kCoWaves * t; }
+  __device__ __forceinline__ int key(int t) const {
+    constexpr int kKeys = L::kFp8 ? 1024 / DT : Geo::kBlkKeys;
+    return blk(t) * kKeys + lane / (64 / kKeys);
+  }
+  __device__ __forceinline__ void init(const Params& p, int D_, int wv_, int lane_) {
+    wv = wv_;
+    lane = lane_;
+    D = D_;
+    constexpr int kElem = L::kFp8 ? 1 : 2;
+    row = (uint32_t)(2 * p.Hkv) * D * kElem;
+#pragma unroll
+    for (int t = 0; t < L::kPerOp; ++t) {
+      const int k = key(t);
+      int ck, cv;  // element columns
+      if constexpr (L::kFp8) {
+        ck = cv = 16 * (lane % (DT / 16));
+      } else {
+        const int pos = lane % (DT / 8);
+        ck = 8 * (pos ^ Geo::xk(k));
+        cv = 32 * ((pos >> 2) ^ Geo::xv(k)) + 8 * (pos & 3);
+      }
+      ck = ck < D ? ck : 0;
+      cv = cv < D ? cv : 0;
+      offk[t] = (uint32_t)k * row + ck * kElem;
+      offv[t] = (uint32_t)k * row + (D + cv) * kElem;
+    }
+  }
 };
 
-template <int MODE>
-__device__ __forceinline__ CoLane co_lane(const Params& p, int wv, int lane) {
-  CoLane c;
-  const uint32_t stride = 2 * p.Hkv * kD;  // elements per key row of the pool
-  if constexpr (MODE == KV_FP8) {
-    c.key[0] = c.key[1] = 8 * wv + (lane >> 3);
-    c.colk[0] = c.colk[1] = 16 * (lane & 7);
-    c.colv[0] = c.colv[1] = kD + 16 * (lane & 7);
-    c.off[0] = c.off[1] = (uint32_t)c.key[0] * stride + c.colk[0];  // (1-byte elements)
-    c.off[2] = c.off[3] = (uint32_t)c.key[0] * stride + c.colv[0];
-    return c;
-  }
-  const int pos = lane & 15;
-#pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int k = 4 * (wv + kCoWaves * t) + (lane >> 4);
-    c.key[t] = k;
-    c.colk[t] = 8 * (pos ^ (k & 15));
-    c.colv[t] = kD + 16 * ((pos >> 1) ^ (k & 7)) + 8 * (pos & 1);
-    c.off[t] = 2 * ((uint32_t)k * stride + c.colk[t]);
-    c.off[2 + t] = 2 * ((uint32_t)k * stride + c.colv[t]);
-  }
-  return c;
-}
-
-// A segment of a tile's chunks whose pages fit the page-id table.
+// A segment of a tile's chunks that fits the table.
 struct CoSeg {
   int c_lo, c_hi;  // chunks
-  int p_lo;        // page of chunk c_lo (table entry 0)
-  int cps;         // chunks per page (page_size / 32)
 };
 
-// This wave's share of chunk c into LDS at dst (wave-uniform LDS address).  bf16: K blocks wv and
-// wv + 4 (keys 4i .. 4i+3 each, 1 KiB per DMA) and the same V blocks into a 16 KiB slot; fp8: K
-// codes of keys 8 wv .. 8 wv + 7 (1 KiB) and their V codes into an 8 KiB code slot.  Keys past
-// kv_len read key kv_len - 1 (scores -inf; V meets P = 0).
-template <int MODE>
-__device__ __forceinline__ void co_issue(const Params& p, const PfTile& tl, const CoLane& cl, const CoSeg& sg,
-                                         const int* ptab, int c, uint32_t dst, int wv, int& err) {
-  int pg = uni(ptab[c / sg.cps - sg.p_lo]);
-  if (pg < 0 || pg >= p.P) {  // out-of-range page id: never dereferenced
-    err |= ERR_PAGE;
-    pg = 0;
+// A row's running maximum before its first visible key: below every score, and finite, so that the
+// exponent of a masked score (-inf) and the first rescale (2^(start - m) = 0) need no special case.
+constexpr float kMaxStart = -1e30f;
+
+// The rows of one 32-row block: row = lane % 32; acc element v of block db is dim
+// 32 db + 8 (v / 4) + 4 (lane / 32) + v % 4; l sums the lane's own 16 keys of each chunk.
+template <int DT>
+struct CoRow {
+  f32x16 acc[DT / 32];
+  float m, l;
+  int pos;  // last visible key of the row
+  bool ok;  // the row exists (token in the tile, pos >= 0)
+};
+
+// The maximum of a value over lanes l and l ^ 32 (the two halves of a row's keys), and the sum.
+__device__ __forceinline__ float halves_max(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return fmaxf(__builtin_bit_cast(float, (unsigned)a[0]), __builtin_bit_cast(float, (unsigned)a[1]));
+}
+__device__ __forceinline__ float halves_sum(float v) {
+  const unsigned u = __builtin_bit_cast(unsigned, v);
+  const auto a = __builtin_amdgcn_permlane32_swap(u, u, false, false);
+  return __builtin_bit_cast(float, (unsigned)a[0]) + __builtin_bit_cast(float, (unsigned)a[1]);
+}
+
+// The tile's chunk stream and compute.  All members are wave-uniform or per-lane registers.
+template <int MODE, int DT, bool UPG>
+struct CoTile {
+  using L = CoLds<MODE, DT, UPG>;
+  using Geo = CoGeo<DT>;
+  const Params& p;
+  const PfTile& tl;
+  CoLoads<MODE, DT, UPG>& ld;
+  uint8_t* lds;
+  CoSeg sg;
+  int n32, hf;                     // lane % 32, lane / 32
+  bf16x8 q[Geo::kSteps];
+  CoRow<DT> st;
+  bf16x8 ka[Geo::kSteps];          // the A fragments of K of chunk c + 1 at the start of step c
+  const uint8_t* vb[3];            // UPG: addresses (base_of) of chunks c + 2 .. c + 4 (fp8 one further)
+  u32x2 ent;                       // UPG: the table entry of the chunk whose K step c issues
+  int c_tail;                      // the chunk with keys past kv_len (-1: none)
+  int plain_to;                    // chunks below it need no masking
+  typedef __attribute__((address_space(3))) const uint8_t* lds_cp;
+  lds_cp kfrag[DT == 256 ? 1 : 2];  // this lane's A fragments in K slot 0 (k-steps 0 and 1)
+  lds_cp vfrag[DT == 256 ? 2 : Geo::kDb];  // its transposing reads in V slot 0 by dim block
+  uint32_t dstk, dstv;              // LDS addresses of this wave's first DMA block of ring slot 0
+
+  static constexpr int kAhead = L::kFp8 ? 1 : 0;  // fp8 chunks are issued one step further ahead
+  __device__ __forceinline__ int last() const { return sg.c_hi - 1; }
+  __device__ __forceinline__ int cl(int c) const { return c < sg.c_hi - 1 ? c : sg.c_hi - 1; }
+
+  // UPG: the table's entry of chunk c (raw, a wave-uniform value in VGPRs) and the address it stands for.
+  __device__ __forceinline__ u32x2 entry(int c) const { return ((const u32x2*)(lds + L::kTable))[c - sg.c_lo]; }
+  __device__ __forceinline__ const uint8_t* base_of(u32x2 e) const {
+    return p.kv + (((uint64_t)(uint32_t)uni((int)e[1]) << 32) | (uint32_t)uni((int)e[0]));
   }
-  const int kmax = tl.kv_len - 1 - c * KV_CHUNK, stride = 2 * p.Hkv * kD;
-  if (kmax >= KV_CHUNK - 1) {  // every key of the chunk exists: a uniform base and the lane's fixed offsets
-    const uint8_t* base = p.kv + kv_elem(p, pg, c * KV_CHUNK, 2 * tl.h) * (MODE == KV_FP8 ? 1 : 2);
-    if constexpr (MODE == KV_FP8) {
-      co_dma_s(base, cl.off[0], dst + 1024u * wv);
-      co_dma_s(base, cl.off[2], dst + 4096u + 1024u * wv);
-    } else {
+
+  // This wave's DMAs of one operand (V: K's rows plus D elements) of chunk c into LDS at dst.  UPG: base is
+  // the chunk's; else rows[t] are the pool rows of the wave's keys.  V of keys past kv_len is read from
+  // key kv_len - 1 (it meets P = 0, so it has to be finite wherever that row is); K of such keys is
+  // whatever their slots of the page hold (their scores are replaced by -inf).
+  // rel: the chunk's number in the segment (mod 4 it names the ring slot; CONST: a compile-time constant).
+  template <bool CONST = true>
+  __device__ __forceinline__ void issue(int rel, int c, bool v, const uint8_t* base, const uint32_t* rows) const {
+    if (L::kOneOp && (ld.wv >= 2) != v) return;
+    constexpr int kStride = L::kFp8 ? kCoWaves * 1024 : 0;
+    const int step = L::kFp8 ? kStride : kCoWaves * (v ? Geo::kVBlk : Geo::kKBlk);
+    const int at = (rel & 3) * (L::kFp8 ? L::kCode : v ? Geo::kVSlot : Geo::kKSlot);
+    const uint32_t dst = (v ? dstv : dstk) + (CONST ? 0 : at);
 #pragma unroll
-      for (int t = 0; t < 2; ++t) {
-        const uint32_t i = (uint32_t)(wv + kCoWaves * t);
-        co_dma_s(base, cl.off[t], dst + 1024u * i);
-        co_dma_s(base, cl.off[2 + t], dst + 8192u + 1024u * i);
+    for (int t = 0; t < L::kPerOp; ++t) {
+      const int imm = (CONST ? at : 0) + step * t;
+      if constexpr (UPG) {
+        co_dma_s(base, v ? (c == c_tail ? ld.offt[t] : ld.offv[t]) : ld.offk[t], dst, imm);
+      } else {
+        const uint32_t col = (v ? ld.offv[t] : ld.offk[t]) - (uint32_t)ld.key(t) * ld.row;
+        co_dma(p.kv + (size_t)rows[t] * ld.row + (size_t)(2 * tl.h) * ld.D * (L::kFp8 ? 1 : 2) + col, dst, imm);
       }
     }
-    return;
   }
-  if constexpr (MODE == KV_FP8) {
-    const uint8_t* base = p.kv + kv_elem(p, pg, c * KV_CHUNK, 2 * tl.h);
-    const uint8_t* row = base + (unsigned)((cl.key[0] < kmax ? cl.key[0] : kmax) * stride);
-    co_dma(row + cl.colk[0], dst + 1024u * wv);
-    co_dma(row + cl.colv[0], dst + 4096u + 1024u * wv);
-    return;
-  }
-  const uint16_t* base = (const uint16_t*)p.kv + kv_elem(p, pg, c * KV_CHUNK, 2 * tl.h);
+  __device__ __forceinline__ void rows_of_chunk(int c, uint32_t rows[L::kPerOp]) const {
+    if constexpr (!UPG) {
+      const uint32_t* tab = (const uint32_t*)(lds + L::kTable) + (c - sg.c_lo) * KV_CHUNK;
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const uint32_t i = (uint32_t)(wv + kCoWaves * t);
-    const uint16_t* row = base + (unsigned)((cl.key[t] < kmax ? cl.key[t] : kmax) * stride);
-    co_dma(row + cl.colk[t], dst + 1024u * i);
-    co_dma(row + cl.colv[t], dst + 8192u + 1024u * i);
-  }
-}
-
-// The pass one step ahead: chunk c's data at src becomes the bf16 slot dst.  Scaled bf16: in place
-// (src == dst), every element times its scale, rounded to bf16 (the layout does not matter);
-// fp8: thread t converts key t / 8, dims 16 (t % 8) .. +15 of K and V with the page's scales into
-// the slot layout (K groups at group ^ (key % 16), V blocks at block ^ (key % 8)).
-template <int MODE>
-__device__ __forceinline__ void co_convert(const Params& p, const CoSeg& sg, const float* scl, int c, const uint8_t* src,
-                                           uint8_t* dst) {
-  const int t = threadIdx.x;
-  if constexpr (MODE == KV_BF16_SCALED) {
-#pragma unroll
-    for (int h = 0; h < 2; ++h) {
-      u32x4* w = (u32x4*)(dst + 8192 * h + 32 * t);
-      const float sc = h ? p.v_scale : p.k_scale;
-      const u32x4 a = w[0], b = w[1];
-      w[0] = scale_bf16x8(a, sc);
-      w[1] = scale_bf16x8(b, sc);
+      for (int t = 0; t < L::kPerOp; ++t) rows[t] = tab[ld.key(t)];
     }
-  } else if constexpr (MODE == KV_FP8) {
-    const int key = t >> 3, g = t & 7, e = 2 * (c / sg.cps - sg.p_lo);
-    const float ks = scl[e], vs = scl[e + 1];
-    const u32x4 kc = *(const u32x4*)(src + key * 128 + 16 * g);
-    const u32x4 vc = *(const u32x4*)(src + 4096 + key * 128 + 16 * g);
-    uint8_t* krow = dst + key * 256;
-    *(u32x4*)(krow + 16 * ((2 * g) ^ (key & 15))) = fp8x8_to_bf16x8(u32x2{kc[0], kc[1]}, ks);
-    *(u32x4*)(krow + 16 * ((2 * g + 1) ^ (key & 15))) = fp8x8_to_bf16x8(u32x2{kc[2], kc[3]}, ks);
-    uint8_t* vblk = dst + 8192 + key * 256 + 32 * (g ^ (key & 7));
-    *(u32x4*)vblk = fp8x8_to_bf16x8(u32x2{vc[0], vc[1]}, vs);
-    *(u32x4*)(vblk + 16) = fp8x8_to_bf16x8(u32x2{vc[2], vc[3]}, vs);
   }
-}
-
-// Where chunk x's data lands (DMA) and where its bf16 slot is read from (compute).
-template <int MODE>
-__device__ __forceinline__ uint8_t* co_land(uint8_t* lds, int x) {
-  return MODE == KV_FP8 ? lds + (x & (kCoSlots - 1)) * kCoCodeSlot : lds + (x & (kCoSlots - 1)) * kCoSlot;
-}
-template <int MODE>
-__device__ __forceinline__ uint8_t* co_slot(uint8_t* lds, int x) {
-  return MODE == KV_FP8 ? lds + kCoSlots * kCoCodeSlot + (x & 1) * kCoSlot : lds + (x & (kCoSlots - 1)) * kCoSlot;
-}
-
-// read_vt_fragments for a slot's V rows (256 bytes at slot + 8192, 32-byte blocks at block ^
-// (key % 8)).
-__device__ __forceinline__ void read_vt_fragments_x(const uint8_t* slot, int n, int j, bf16x8 va[8]) {
-  typedef __attribute__((address_space(3))) short4_t* lds_s4;
-  const int k = 4 * j + (n >> 2), x = k & 7;  // key of the low half; the high half (k + 16) has the same k % 8
-  const uint8_t* vb = slot + 8192 + k * 256 + 8 * (n & 3);
-#pragma unroll
-  for (int d = 0; d < 8; ++d) {
-    const int off = 32 * (d ^ x);
-    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(vb + off));
-    const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(vb + 16 * 256 + off));
-    va[d] = __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  // Where a chunk's K / V data land, and where their bf16 slots are read (rel as in issue).
+  __device__ __forceinline__ uint8_t* land(int rel, bool v) const {
+    if constexpr (L::kFp8) return lds + (v ? L::kCodeV : 0) + (rel & 3) * L::kCode;
+    return slot(rel, v);
   }
-}
+  static __device__ __forceinline__ constexpr int slot_at(int rel, bool v) {
+    return (rel & (L::kSlots - 1)) * (v ? Geo::kVSlot : Geo::kKSlot);
+  }
+  __device__ __forceinline__ uint8_t* slot(int rel, bool v) const { return lds + (v ? L::kV : L::kK) + slot_at(rel, v); }
+  // Issue one operand of the segment's chunk rel outside the loop.
+  template <int REL, bool V>
+  __device__ __forceinline__ void issue_at() {
+    const int c = cl(sg.c_lo + REL);
+    uint32_t rows[L::kPerOp];
+    const uint8_t* base = nullptr;
+    if constexpr (UPG) base = base_of(entry(c));
+    rows_of_chunk(c, rows);
+    issue(REL, c, V, base, rows);
+  }
 
-// S = K Q^T of chunk slot buf for the wave's two row blocks: the eight K fragment reads go out
-// together, then the sixteen MFMAs.
-__device__ __forceinline__ void co_qk(const uint8_t* buf, const bf16x8 q[2][4], f32x4 sc[2][2], int n, int j) {
+  // The pass over one operand of chunk c (see the section comment).  Every element goes to the same
+  // place of its slot whatever its scale; c may lie past the segment (clamped data, never used).
+  __device__ __forceinline__ void convert(int rel, int c, bool v) const {
+    const int t = threadIdx.x;
+    if constexpr (MODE == KV_BF16_SCALED) {
+      constexpr int kBytes = KV_CHUNK * Geo::kRow / 256;  // per thread
+      const int at = kBytes * t, blk = at >> 10, in = at & 1023;
+      uint8_t* b = slot(rel, v) + blk * (v ? Geo::kVBlk : Geo::kKBlk) + in;
+      const float sc = v ? p.v_scale : p.k_scale;
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) sc[rb][0] = sc[rb][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-  bf16x8 a[4][2];
+      for (int i = 0; i < kBytes / 16; ++i) *(u32x4*)(b + 16 * i) = scale_bf16x8(*(const u32x4*)(b + 16 * i), sc);
+    } else if constexpr (MODE == KV_FP8) {
+      constexpr int kLanes = DT / 16;             // 16-code pieces of a key
+      constexpr int kPieces = KV_CHUNK * kLanes;  // of the chunk: 128 (DT 64), 256 or 512
 #pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) a[s][kb] = *(const bf16x8*)(buf + (16 * kb + n) * 256 + 16 * ((4 * s + j) ^ n));
-#pragma unroll
-  for (int s = 0; s < 4; ++s)
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      sc[0][kb] = mfma(a[s][kb], q[0][s], sc[0][kb]);
-      sc[1][kb] = mfma(a[s][kb], q[1][s], sc[1][kb]);
+      for (int i0 = 0; i0 < kPieces; i0 += 256) {
+        const int i = (i0 + t) & (kPieces - 1);  // (DT 64: two threads write each piece alike)
+        const int key = i / kLanes, g = i % kLanes;
+        const u32x4 w = *(const u32x4*)(land(rel, v) + 16 * i);
+        const float* sc = (const float*)(lds + L::kScale);
+        u32x4 lo, hi;
+        if (UPG && !v) {  // exact: the scale multiplies the scores
+          lo = fp8x8_to_bf16x8_exact(u32x2{w[0], w[1]});
+          hi = fp8x8_to_bf16x8_exact(u32x2{w[2], w[3]});
+        } else {
+          const int cc = cl(c);
+          const int e = UPG ? cc - sg.c_lo : (cc - sg.c_lo) * KV_CHUNK + key;
+          const float s = sc[2 * e + (v ? 1 : 0)];
+          lo = fp8x8_to_bf16x8(u32x2{w[0], w[1]}, s);
+          hi = fp8x8_to_bf16x8(u32x2{w[2], w[3]}, s);
+        }
+        uint8_t* b = slot(rel, v) + (key / Geo::kBlkKeys) * (v ? Geo::kVBlk : Geo::kKBlk) +
+                     (key % Geo::kBlkKeys) * Geo::kRow;
+        if (v) {
+          uint8_t* d = b + 64 * ((g >> 1) ^ Geo::xv(key)) + 32 * (g & 1);
+          *(u32x4*)d = lo;
+          *(u32x4*)(d + 16) = hi;
+        } else {
+          *(u32x4*)(b + 16 * ((2 * g) ^ Geo::xk(key))) = lo;
+          *(u32x4*)(b + 16 * ((2 * g + 1) ^ Geo::xk(key))) = hi;
+        }
+      }
     }
-  __builtin_amdgcn_sched_group_barrier(0x100, 8, 0);
-  __builtin_amdgcn_sched_group_barrier(0x008, 16, 0);
-}
-
-// Softmax and O += P V of chunk slot buf, the V^T fragments read before the softmax.
-template <bool PLAIN>
-__device__ __forceinline__ void co_pv(const Params& p, const PfTile& tl, int c, const uint8_t* buf, const f32x4 sc[2][2],
-                                      PfRow st[2], int n, int j) {
-  bf16x8 va[8];
-  read_vt_fragments_x(buf, n, j, va);
-  bf16x8 pb0, pb1;
-  if constexpr (PLAIN) {
-    float m0 = pf_lane_max(sc[0]), m1 = pf_lane_max(sc[1]);
-    rows4_max2(m0, m1);  // both row blocks' row maxima in three swaps
-    pb0 = pf_softmax_plain_m(p, sc[0], st[0], m0);
-    pb1 = pf_softmax_plain_m(p, sc[1], st[1], m1);
-  } else {
-    pb0 = pf_softmax(p, tl, c, sc[0], st[0], j);
-    pb1 = pf_softmax(p, tl, c, sc[1], st[1], j);
   }
+
+  __device__ __forceinline__ bf16x8 k_fragment(int rel, int s) const {
+    typedef __attribute__((address_space(3))) const bf16x8* lds_b8;
+    if constexpr (DT == 256) return *(lds_b8)(kfrag[0] + slot_at(rel, false) + 32 * s);
+    return *(lds_b8)(kfrag[s & 1] + slot_at(rel, false) + 64 * (s >> 1));
+  }
+  __device__ __forceinline__ bf16x8 v_fragment(int rel, int db, int t) const {
+    typedef __attribute__((address_space(3))) short4_t* lds_s4;
+    // keys 16t + 8 lh + ..: whole blocks further
+    constexpr int kStep = (8 / Geo::kBlkKeys) * Geo::kVBlk;
+    const lds_cp b = (DT == 256 ? vfrag[db & 1] + 128 * (db >> 1) : vfrag[db]) + slot_at(rel, true) + 2 * t * kStep;
+    const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)b);
+    const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(b + kStep));
+    return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
+  }
+  __device__ __forceinline__ void init_fragments(int lane) {
+    n32 = lane & 31;
+    hf = lane >> 5;
+    const lds_cp kr = (lds_cp)(lds + L::kK) + (n32 / Geo::kBlkKeys) * Geo::kKBlk + (n32 % Geo::kBlkKeys) * Geo::kRow;
+    if constexpr (DT == 256) {
+      kfrag[0] = kr + 16 * (hf ^ Geo::xk(n32));
+    } else {
+      kfrag[0] = kr + 16 * (hf ^ Geo::xk(n32));
+      kfrag[1] = kr + 16 * ((2 + hf) ^ Geo::xk(n32));
+    }
+    // lane nn of group (hf, dsub) addresses key 4 hf + nn / 4, dims 16 dsub + 4 (nn % 4) .. of a block
+    const int nn = lane & 15, dsub = (lane >> 4) & 1, k0 = 4 * hf + (nn >> 2);
+    const lds_cp vr = (lds_cp)(lds + L::kV) + (k0 / Geo::kBlkKeys) * Geo::kVBlk + (k0 % Geo::kBlkKeys) * Geo::kRow +
+                      32 * dsub + 8 * (nn & 3);
 #pragma unroll
-  for (int d = 0; d < 8; ++d) {
-    st[0].acc[d] = mfma(va[d], pb0, st[0].acc[d]);
-    st[1].acc[d] = mfma(va[d], pb1, st[1].acc[d]);
+    for (int d = 0; d < (DT == 256 ? 2 : Geo::kDb); ++d) vfrag[d] = vr + 64 * (d ^ Geo::xv(k0));
+    const int w = ld.blk(0);
+    dstk = uni((int)(lds_addr_of(lds + (L::kFp8 ? 0 : L::kK)) + (uint32_t)w * (L::kFp8 ? 1024 : Geo::kKBlk)));
+    dstv = uni((int)(lds_addr_of(lds + (L::kFp8 ? L::kCodeV : L::kV)) + (uint32_t)w * (L::kFp8 ? 1024 : Geo::kVBlk)));
   }
-}
 
-// Step on chunk c of segment sg.  In flight on entry: the DMAs of c, c + 1, c + 2.  Wait (bf16: for
-// this wave's DMAs of c; converting modes: of c + 1, c having been converted by the previous step),
-// barrier (every wave's share is in LDS, the previous step's conversion visible, and every wave done
-// with chunk c - 1's slot); converting modes: chunk c + 1's pass; S = K Q^T of c; the DMAs of c + 3
-// into the freed ring slot (issued while the MFMAs run); the softmax and P V of c.
-template <int MODE, bool PLAIN>
-__device__ __forceinline__ void co_step(const Params& p, const PfTile& tl, const CoLane& cl, const CoSeg& sg,
-                                        const int* ptab, const float* scl, int c, uint8_t* lds, const bf16x8 q[2][4],
-                                        PfRow st[2], int wv, int n, int j, int& err) {
-  const int last = sg.c_hi - 1;
-  co_barrier<(co_converts<MODE>() ? 1 : 2) * co_dmas<MODE>()>();
-  if constexpr (co_converts<MODE>()) {
-    const int cn = c + 1 < last ? c + 1 : last;
-    co_convert<MODE>(p, sg, scl, cn, co_land<MODE>(lds, c + 1), co_slot<MODE>(lds, c + 1));
+  // O += P V of the segment's chunk rel (epilogue).
+  __device__ __forceinline__ void add_pv(int rel, const bf16x8 pv[2]) {
+#pragma unroll
+    for (int t = 0; t < 2; ++t)
+#pragma unroll
+      for (int db = 0; db < Geo::kDb; ++db) st.acc[db] = mfma32(v_fragment(rel, db, t), pv[t], st.acc[db]);
   }
-  const uint8_t* buf = co_slot<MODE>(lds, c);
-  f32x4 sc[2][2];
-  co_qk(buf, q, sc, n, j);
-  const int cn = c + 3 < last ? c + 3 : last;
-  co_issue<MODE>(p, tl, cl, sg, ptab, cn, lds_addr_of(co_land<MODE>(lds, c + 3)), wv, err);
-  co_pv<PLAIN>(p, tl, c, buf, sc, st, n, j);
-}
+
+  // Step on chunk c.  In: s = S of chunk c, pv = P of chunk c - 1, ka = K of chunk c + 1.  Out: s_next = S
+  // of chunk c + 1, p_new = P of chunk c, ka = K of chunk c + 2.  In LDS on entry (after the barrier): K of
+  // c + 2, V of c - 1 (converting modes: also K of c + 3 and V of c, unconverted).  Issues K of c + 5 and
+  // V of c + 2 (fp8: one further).  The K fragments are a step ahead so that MFMAs can issue right after
+  // the barrier, over the V reads' latency and the DMAs' address work.
+  // R: c - c_lo modulo 4 (the ring slots become constants of each copy), or -1: not known.
+  template <bool PLAIN, int R>
+  __device__ __forceinline__ void step(int c, const f32x16& s, f32x16& s_next, const bf16x8 pv[2], bf16x8 p_new[2]) {
+    const int r = R >= 0 ? R : c - sg.c_lo;
+    const int ck = cl(c + 5 + kAhead), cv = cl(c + 2 + kAhead);
+    uint32_t rk[L::kPerOp], rv[L::kPerOp];
+    rows_of_chunk(ck, rk);
+    rows_of_chunk(cv, rv);
+    float sl2 = p.scale_log2, ksc = 1.f;
+    if constexpr (L::kFp8 && UPG) ksc = ((const float*)(lds + L::kScale))[2 * (c - sg.c_lo)];
+    // bf16 waits for K of c + 2 and V of c - 1 (issued three steps ago), scaled for K of c + 3 and V of c
+    // (two), fp8 for the same (three)
+    co_barrier<(MODE == KV_BF16_SCALED ? 1 : 2) * L::kStepDmas>();
+    const uint8_t* bk = nullptr;
+    if constexpr (UPG) bk = base_of(ent);
+    if constexpr (L::kFp8 && UPG) sl2 *= uni_f(ksc);
+
+    // softmax of chunk c (exp2 domain, lazily moved reference: see unit_softmax), as work items: the row
+    // maximum (0..2), the probabilities (3..18), their sum (19, 20) and P (21, 22)
+    constexpr int kItems = 23;
+    float x[16], e[16], ma, mb, mn, sum;
+    bool grow;
+    auto score = [&](int i) { return PLAIN ? s[i] : x[i]; };
+    auto max3 = [&](int i) { return fmaxf(fmaxf(score(i), score(i + 1)), score(i + 2)); };
+    auto item = [&](int it) {
+      if (it == 0) {
+        ma = fmaxf(fmaxf(max3(0), score(3)), score(4));
+        mb = fmaxf(fmaxf(max3(5), score(8)), score(9));
+      } else if (it == 1) {
+        ma = fmaxf(fmaxf(ma, score(10)), score(11));
+        mb = fmaxf(fmaxf(mb, score(12)), score(13));
+        ma = fmaxf(fmaxf(ma, score(14)), score(15));
+      } else if (it == 2) {
+        ma = halves_max(fmaxf(ma, mb));
+        const float mc = PLAIN ? ma * sl2 : ma;
+        grow = mc > st.m + kRescaleLog2;
+        mn = grow ? mc : st.m;
+      } else if (it < 19) {
+        const int i = it - 3;
+        e[i] = __builtin_amdgcn_exp2f(PLAIN ? __builtin_fmaf(s[i], sl2, -mn) : x[i] - mn);
+      } else if (it == 19) {
+        sum = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+      } else if (it == 20) {
+        sum += ((e[8] + e[9]) + (e[10] + e[11])) + ((e[12] + e[13]) + (e[14] + e[15]));
+      } else {
+        const int t = it - 21;
+        u32x4 w;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) w[i] = pack_bf16x2(e[8 * t + 2 * i], e[8 * t + 2 * i + 1]);
+        p_new[t] = __builtin_bit_cast(bf16x8, w);
+      }
+    };
+    if constexpr (!PLAIN) {
+      const int key0 = c * KV_CHUNK + 4 * hf;
+      if (c < plain_to) {
+#pragma unroll
+        for (int i = 0; i < 16; ++i) x[i] = s[i] * sl2;
+      } else {
+        // soft_cap * tanh(t / soft_cap) with tanh(y) = sign(y) (1 - z) / (1 + z), z = exp(-2 |y|)
+        const float sm = L::kFp8 && UPG ? p.sm_scale * uni_f(ksc) : p.sm_scale;
+        const float ec = p.soft_cap > 0.f ? -2.f * kLog2e * sm / p.soft_cap : 0.f;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+          float xv = s[i] * sl2;
+          if (p.soft_cap > 0.f) {
+            const float z = __builtin_amdgcn_exp2f(-fabsf(s[i] * ec));
+            xv = copysignf(p.soft_cap * kLog2e * ((1.f - z) / (1.f + z)), s[i] * sm);
+          }
+          const int kt = key0 + 8 * (i >> 2) + (i & 3);
+          const bool masked = kt > st.pos || (p.sliding_window > 0 && kt <= st.pos - p.sliding_window);
+          if (masked) xv += p.mask_log2;
+          if (kt >= tl.kv_len) xv = -INFINITY;
+          x[i] = xv;
+        }
+      }
+    }
+
+    // One MFMA, then a share of the softmax, fenced from the next pair: a wave issues in order, so an MFMA
+    // behind another stalls it for the matrix cores' 32 cycles, in which these VALU instructions run.
+    // (Left to itself the scheduler puts the MFMAs together, and the two kinds run one after the other.)
+    constexpr int kPairs = Geo::kSteps + 2 * Geo::kDb;
+    bf16x8 va[2][Geo::kDb], kn[Geo::kSteps];
+    s_next = f32x16{};
+#pragma unroll
+    for (int g = 0; g < kPairs; ++g) {
+      const int pg = g - Geo::kSteps;  // P V products follow those of S
+      if (g < Geo::kSteps)
+        s_next = mfma32(ka[g], q[g], s_next);
+      else
+        st.acc[pg % Geo::kDb] = mfma32(va[pg / Geo::kDb][pg % Geo::kDb], pv[pg / Geo::kDb], st.acc[pg % Geo::kDb]);
+      if (g == 0) {
+#pragma unroll
+        for (int db = 0; db < Geo::kDb; ++db) va[0][db] = v_fragment(r + 3, db, 0);
+      }
+      if (g == 1) issue<(R >= 0)>(r + 5 + kAhead, ck, false, bk, rk);
+      if (g == 2) issue<(R >= 0)>(r + 2 + kAhead, cv, true, vb[0], rv);
+      // the second half's V fragments and the next K fragments take the registers of the fragments used up
+      if (g == Geo::kSteps - 1) {
+#pragma unroll
+        for (int db = 0; db < Geo::kDb; ++db) va[1][db] = v_fragment(r + 3, db, 1);
+      }
+      if (g == Geo::kSteps) {
+#pragma unroll
+        for (int i = 0; i < Geo::kSteps / 2; ++i) kn[i] = k_fragment(r + 2, i);
+      }
+      if (g == Geo::kSteps + Geo::kDb) {
+#pragma unroll
+        for (int i = Geo::kSteps / 2; i < Geo::kSteps; ++i) kn[i] = k_fragment(r + 2, i);
+      }
+#pragma unroll
+      for (int it = 0; it < kItems; ++it)
+        if (it >= (g * kItems) / kPairs && it < ((g + 1) * kItems) / kPairs) item(it);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int i = 0; i < Geo::kSteps; ++i) ka[i] = kn[i];
+    if constexpr (UPG) {
+      vb[0] = vb[1];
+      vb[1] = vb[2];
+      vb[2] = bk;
+      ent = entry(cl(c + 6 + kAhead));
+    }
+    {  // all of it is made here: the compiler would sink what only later steps use below the branch
+      u32x4 w0 = __builtin_bit_cast(u32x4, p_new[0]), w1 = __builtin_bit_cast(u32x4, p_new[1]);
+      asm volatile("" : "+v"(w0), "+v"(w1), "+v"(sum));
+      p_new[0] = __builtin_bit_cast(bf16x8, w0);
+      p_new[1] = __builtin_bit_cast(bf16x8, w1);
+    }
+    if constexpr (co_converts<MODE>()) {  // visible to the next step's barrier
+      convert(r + 3, c + 3, false);
+      convert(r, c, true);
+    }
+    if (__ballot(grow)) {  // acc holds P V up to chunk c - 1, against the old reference
+      const float alpha = __builtin_amdgcn_exp2f(st.m - mn);
+      st.l *= alpha;
+#pragma unroll
+      for (int db = 0; db < Geo::kDb; ++db) st.acc[db] *= alpha;
+    }
+    st.m = mn;
+    st.l += sum;
+  }
+  static __device__ __forceinline__ float uni_f(float v) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, v)));
+  }
+
+  // The segment sg: fill its table, prime the rings, run its chunks (those below cp plain).
+  __device__ __forceinline__ void run_segment(int cp, int& err, TlAcc& ta) {
+    RPA_TL(const long long tl_a = tl_clock();)
+    __syncthreads();  // the previous segment's or tile's tables and slots are no longer read
+    uint32_t* tab = (uint32_t*)(lds + L::kTable);
+    float* scl = (float*)(lds + L::kScale);
+    bool plain_ok = true;  // every K scale of the segment is positive: it commutes with the row maximum
+    const int nent = (sg.c_hi - sg.c_lo) * (UPG ? 1 : KV_CHUNK);
+    for (int t = threadIdx.x; t < nent; t += kCoWaves * 64) {
+      int kt = sg.c_lo * KV_CHUNK + (UPG ? t * KV_CHUNK : t);
+      kt = kt < tl.kv_len ? kt : tl.kv_len - 1;
+      int pg = p.page_indices[(size_t)tl.seq * p.PPS + page_of(kt, p)];
+      if (pg < 0 || pg >= p.P) {  // out-of-range page id: never dereferenced
+        err |= ERR_PAGE;
+        pg = 0;
+      }
+      if constexpr (UPG)
+        ((uint64_t*)tab)[t] = kv_elem(p, pg, kt, 2 * tl.h, ld.D) * (L::kFp8 ? 1 : 2);
+      else
+        tab[t] = (uint32_t)pg * (uint32_t)p.S + (uint32_t)slot_of(kt, p);
+      if constexpr (L::kFp8) {  // the page's K and V scales of kv head h
+        f32x2 sv = f32x2{1.f, 1.f};  // times the scalar k_scale / v_scale, as the decode role applies them
+        if (p.kv_scales) sv = *(const f32x2*)(p.kv_scales + ((size_t)pg * p.Hkv + tl.h) * 2);
+        *(f32x2*)(scl + 2 * t) = f32x2{sv[0] * p.k_scale, sv[1] * p.v_scale};
+        plain_ok = plain_ok && sv[0] * p.k_scale > 0.f;
+      }
+    }
+    if constexpr (L::kFp8 && UPG) {
+      const int bad = __ballot(!plain_ok) != 0;
+      if ((threadIdx.x & 63) == 0) ((int*)(lds + L::kFlags))[threadIdx.x >> 6] = bad;
+    }
+    const int c0 = sg.c_lo;
+    {  // V "of chunk c0 - 1" meets P = 0 in the first step: any finite values do
+      uint8_t* z = slot(3, true);
+      for (int i = threadIdx.x * 16; i < Geo::kVSlot; i += kCoWaves * 64 * 16) *(u32x4*)(z + i) = u32x4{0u, 0u, 0u, 0u};
+    }
+    // the tables and (first segment) the queries have landed, on every path: the compiler then has
+    // no load of its own left to wait for inside the step loop
+    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
+    __syncthreads();
+    // the order the waits count on: K of c0 .. c0 + 2 first, then what the steps expect in flight
+    issue_at<0, false>();
+    issue_at<1, false>();
+    issue_at<2, false>();
+    issue_at<3, false>();
+    issue_at<0, true>();
+    co_barrier<L::kOneOp ? 0 : 2 * L::kPerOp>();
+    if constexpr (co_converts<MODE>()) {
+      convert(0, c0, false);
+      convert(1, c0 + 1, false);
+      if constexpr (!L::kFp8) convert(2, c0 + 2, false);
+      asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    }
+    f32x16 sa = {}, sb;
+#pragma unroll
+    for (int i = 0; i < Geo::kSteps; ++i) sa = mfma32(k_fragment(0, i), q[i], sa);
+#pragma unroll
+    for (int i = 0; i < Geo::kSteps; ++i) ka[i] = k_fragment(1, i);
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");  // K of c0 (and its codes) is free
+    if constexpr (L::kFp8) convert(2, c0 + 2, false);
+    issue_at<4, false>();
+    issue_at<1, true>();
+    if constexpr (L::kFp8) {
+      issue_at<5, false>();
+      issue_at<2, true>();
+    }
+    if constexpr (UPG) {
+#pragma unroll
+      for (int i = 0; i < 3; ++i) vb[i] = base_of(entry(cl(c0 + 2 + kAhead + i)));
+      ent = entry(cl(c0 + 5 + kAhead));
+    }
+    bf16x8 pa[2], pb[2];
+    pa[0] = pa[1] = bf16x8{};
+    plain_to = cp;
+    if constexpr (L::kFp8 && UPG) {  // a K scale that is not positive: the plain path's maximum would not hold
+      const int4 bad = *(const int4*)(lds + L::kFlags);
+      if (uni(bad.x | bad.y | bad.z | bad.w)) plain_to = c0;
+    }
+    const int cpe = plain_to < sg.c_hi ? plain_to : sg.c_hi;
+    int c = c0;
+    RPA_TL(const long long tl_b = tl_clock(); ta.setup += tl_b - tl_a;)
+    for (; c + 4 <= cpe; c += 4) {
+      step<true, 0>(c, sa, sb, pa, pb);
+      step<true, 1>(c + 1, sb, sa, pb, pa);
+      step<true, 2>(c + 2, sa, sb, pa, pb);
+      step<true, 3>(c + 3, sb, sa, pb, pa);
+    }
+    for (; c < sg.c_hi; ++c) {
+      step<false, -1>(c, sa, sb, pa, pb);
+      sa = sb;
+      pa[0] = pb[0];
+      pa[1] = pb[1];
+    }
+    co_barrier<0>();  // V of the last chunk (and the clamped DMAs past the segment) have landed
+    add_pv(last() - c0, pa);
+    RPA_TL(ta.loop += tl_clock() - tl_b;)
+  }
+};
 
 // slot >= 0: the tile is one part of a split tile, its (m, l, acc) go to that partial slot
-template <int MODE>
-__device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, const CoLane& cln, uint8_t* lds, int wv,
-                                        int lane, int n, int j, int& err, int slot, TlAcc& ta) {
-  RPA_TL(const long long tl_a = tl_clock(); long long tl_b = 0;)
-  PfRow st[2];
-  bf16x8 q[2][4];
+template <int MODE, int DT, bool UPG>
+__device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoads<MODE, DT, UPG>& ld,
+                                        uint8_t* lds, int wv, int lane, int& err, int slot, TlAcc& ta) {
+  using L = CoLds<MODE, DT, UPG>;
+  using Geo = CoGeo<DT>;
+  const int D = ld.D;
+  CoTile<MODE, DT, UPG> x{p, tl, ld, lds};
+  x.init_fragments(lane);
+  const int hf = x.hf, r = 32 * wv + x.n32;
+  const int tok = r / p.G, g = r - tok * p.G;
+  x.st.pos = tl.kv_len - tl.q_len + tl.tok0 + tok;
+  x.st.ok = tok < tl.ntok && x.st.pos >= 0;
+  {
+    const int qtok = x.st.ok ? tl.q_start + tl.tok0 + tok : tl.q_start;
+    const uint16_t* qp = p.q + ((size_t)qtok * p.Hq + tl.h * p.G + (x.st.ok ? g : 0)) * D;
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const int r = 32 * wv + 16 * rb + n;
-    const int tok = r / p.G, g = r - tok * p.G;
-    st[rb].ok = tok < tl.ntok;
-    st[rb].pos = tl.kv_len - tl.q_len + tl.tok0 + tok;
-    st[rb].ok = st[rb].ok && st[rb].pos >= 0;
-    const int qtok = st[rb].ok ? tl.q_start + tl.tok0 + tok : tl.q_start;
-    const uint16_t* qp = p.q + ((size_t)qtok * p.Hq + tl.h * p.G + (st[rb].ok ? g : 0)) * kD + 8 * j;
+    for (int s = 0; s < Geo::kSteps; ++s) {  // a narrow row's dims past D are zero
+      const int d = 16 * s + 8 * hf;
+      const u32x4 w = *(const u32x4*)(qp + (d < D ? d : 0));
+      x.q[s] = __builtin_bit_cast(bf16x8, d < D ? w : u32x4{0u, 0u, 0u, 0u});
+    }
+  }
 #pragma unroll
-    for (int s = 0; s < 4; ++s) q[rb][s] = *(const bf16x8*)(qp + 32 * s);
+  for (int d = 0; d < Geo::kDb; ++d) x.st.acc[d] = f32x16{};
+  x.st.m = kMaxStart;
+  x.st.l = 0.f;
+  {
+    const int kmax = (tl.kv_len - 1) % KV_CHUNK;  // last key of the sequence's last chunk
+    x.c_tail = kmax < KV_CHUNK - 1 ? (tl.kv_len - 1) / KV_CHUNK : -1;
 #pragma unroll
-    for (int d = 0; d < 8; ++d) st[rb].acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
-    st[rb].m = -INFINITY;
-    st[rb].l = 0.f;
+    for (int t = 0; t < L::kPerOp; ++t) {
+      const int k = ld.key(t);
+      ld.offt[t] = ld.offv[t] - (uint32_t)(k > kmax ? k - kmax : 0) * ld.row;
+    }
   }
   // chunks below cp are seen in full by every row (the plain softmax); the rest (the diagonal, a
   // window, a soft cap, masked keys of a finite mask value) take the general one
@@ -2346,130 +2686,104 @@ __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, const
     cp = (pos_min + 1) / KV_CHUNK;
     cp = cp < tl.kv_len / KV_CHUNK ? cp : tl.kv_len / KV_CHUNK;
   }
-  int* ptab = (int*)(lds + kCoPageBase);
-  float* scl = (float*)(lds + kCoScaleBase);
-  CoSeg sg;
-  sg.cps = p.S / KV_CHUNK;
-  for (sg.c_lo = tl.c_lo; sg.c_lo < tl.c_hi; sg.c_lo = sg.c_hi) {
-    sg.p_lo = sg.c_lo / sg.cps;
-    sg.c_hi = (sg.p_lo + kCoPages) * sg.cps;
-    sg.c_hi = sg.c_hi < tl.c_hi ? sg.c_hi : tl.c_hi;
-    const int npg = (sg.c_hi - 1) / sg.cps - sg.p_lo + 1;
-    __syncthreads();  // the previous segment's or tile's tables and slots are no longer read
-    for (int t = threadIdx.x; t < npg; t += kCoWaves * 64) {
-      const int pg = p.page_indices[(size_t)tl.seq * p.PPS + sg.p_lo + t];
-      ptab[t] = pg;
-      if constexpr (MODE == KV_FP8) {  // the page's K and V scales of kv head h (page 0's for a bad id)
-        f32x2 sv = f32x2{1.f, 1.f};  // times the scalar k_scale / v_scale, as the decode role applies them
-        if (p.kv_scales) sv = *(const f32x2*)(p.kv_scales + ((size_t)(pg >= 0 && pg < p.P ? pg : 0) * p.Hkv + tl.h) * 2);
-        *(f32x2*)(scl + 2 * t) = f32x2{sv[0] * p.k_scale, sv[1] * p.v_scale};
-      }
-    }
-    // the tables and (first segment) the queries have landed, on every path: the compiler then has
-    // no load of its own left to wait for inside the step loop
-    __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
-    __syncthreads();
-    const int c0 = sg.c_lo, last = sg.c_hi - 1;
-    auto cl = [&](int c) { return c < last ? c : last; };
-#pragma unroll
-    for (int k = 0; k < 3; ++k)
-      co_issue<MODE>(p, tl, cln, sg, ptab, cl(c0 + k), lds_addr_of(co_land<MODE>(lds, c0 + k)), wv, err);
-    if constexpr (co_converts<MODE>()) {  // chunk c0's pass before the loop takes over
-      co_barrier<2 * co_dmas<MODE>()>();
-      co_convert<MODE>(p, sg, scl, c0, co_land<MODE>(lds, c0), co_slot<MODE>(lds, c0));
-    }
-    int c = c0;
-    RPA_TL(if (tl_b == 0) tl_b = tl_clock();)
-    const int cpe = cp < sg.c_hi ? cp : sg.c_hi;
-    for (; c < cpe; ++c) co_step<MODE, true>(p, tl, cln, sg, ptab, scl, c, lds, q, st, wv, n, j, err);
-    for (; c < sg.c_hi; ++c) co_step<MODE, false>(p, tl, cln, sg, ptab, scl, c, lds, q, st, wv, n, j, err);
-    co_drain();  // the clamped DMAs past the segment land before the slots are reused
+  for (x.sg.c_lo = tl.c_lo; x.sg.c_lo < tl.c_hi; x.sg.c_lo = x.sg.c_hi) {
+    x.sg.c_hi = x.sg.c_lo + L::kSegChunks;
+    x.sg.c_hi = x.sg.c_hi < tl.c_hi ? x.sg.c_hi : tl.c_hi;
+    x.run_segment(cp, err, ta);
   }
-  RPA_TL(const long long tl_c = tl_clock(); ta.setup += tl_b - tl_a; ta.loop += tl_c - tl_b; ta.tiles += 1;
-         ta.steps += tl.c_hi - tl.c_lo;)
+  RPA_TL(const long long tl_c = tl_clock(); ta.tiles += 1; ta.steps += tl.c_hi - tl.c_lo;)
 
+  CoRow<DT>& st = x.st;
+  const float lt = halves_sum(st.l);
   if (slot >= 0) {  // a part of a split tile: its unnormalised state, (m, l) in log2 units
-#pragma unroll
-    for (int rb = 0; rb < 2; ++rb) {
-      const float lt = rows4_sum(st[rb].l);
-      if (!st[rb].ok) continue;
-      const int r = 32 * wv + 16 * rb + n;
+    if (st.ok) {
       float* ml = p.pk_ml + ((size_t)slot * 128 + r) * 2;
-      if (j == 0) *(f32x2*)ml = f32x2{st[rb].m, lt};
-      float* acc = p.pk_acc + ((size_t)slot * 128 + r) * kD + 4 * j;
+      if (hf == 0) *(f32x2*)ml = f32x2{st.m, lt};
+      float* acc = p.pk_acc + ((size_t)slot * 128 + r) * kD + 4 * hf;
 #pragma unroll
-      for (int d = 0; d < 8; ++d) *(f32x4*)(acc + 16 * d) = st[rb].acc[d];
+      for (int d = 0; d < Geo::kDb; ++d)
+#pragma unroll
+        for (int a = 0; a < 4; ++a)
+          *(f32x4*)(acc + 32 * d + 8 * a) =
+              f32x4{st.acc[d][4 * a], st.acc[d][4 * a + 1], st.acc[d][4 * a + 2], st.acc[d][4 * a + 3]};
     }
     RPA_TL(ta.write += tl_clock() - tl_c;)
     return;
   }
+  // a lane holds dims 8a + 4 hf .. +3 of each 32-dim block: one v_permlane32_swap of two such pieces
+  // gives the lower half dims 8a .. 8a+7 and the upper half the next eight -- 16-byte stores.  (The
+  // swaps need every lane; only the stores are predicated.)
+  const float inv = 1.f / lt;
+  uint16_t* op = p.out + ((size_t)(tl.q_start + tl.tok0 + (st.ok ? tok : 0)) * p.Hq + tl.h * p.G + (st.ok ? g : 0)) * D;
 #pragma unroll
-  for (int rb = 0; rb < 2; ++rb) {
-    const float lt = rows4_sum(st[rb].l);
-    if (!st[rb].ok) continue;
-    const int r = 32 * wv + 16 * rb + n;
-    const int tok = r / p.G, g = r - tok * p.G;
-    const float inv = 1.f / lt;
-    uint16_t* op = p.out + ((size_t)(tl.q_start + tl.tok0 + tok) * p.Hq + tl.h * p.G + g) * kD + 4 * j;
+  for (int d = 0; d < Geo::kDb; ++d)
 #pragma unroll
-    for (int d = 0; d < 8; ++d) {
-      u32x2 w;
-      w[0] = pack_bf16x2(st[rb].acc[d][0] * inv, st[rb].acc[d][1] * inv);
-      w[1] = pack_bf16x2(st[rb].acc[d][2] * inv, st[rb].acc[d][3] * inv);
-      *(u32x2*)(op + 16 * d) = w;
+    for (int a = 0; a < 4; a += 2) {
+      uint32_t w[2][2];
+#pragma unroll
+      for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int e = 0; e < 2; ++e)
+          w[i][e] = pack_bf16x2(st.acc[d][4 * (a + i) + 2 * e] * inv, st.acc[d][4 * (a + i) + 2 * e + 1] * inv);
+      const auto s0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
+      const auto s1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
+      const int dim = 32 * d + 8 * (a + hf);
+      if (st.ok && dim < D)
+        *(u32x4*)(op + dim) = u32x4{(unsigned)s0[0], (unsigned)s1[0], (unsigned)s0[1], (unsigned)s1[1]};
     }
-  }
   RPA_TL(ta.write += tl_clock() - tl_c;)
 }
 
 // The (sequence, token block) pairs of the call's prefill tiles in queue order (sequences in window
-// order, each sequence's token blocks last first), held per lane: lane l's sequence of window w
-// owns pairs base[w] + off[w] .. + nt[w] - 1.  One DPP scan per window; a pair's tile then costs
-// a ballot and a few readlanes (co_tile_of), not a scan.
-struct CoPairs {
-  int off[4], nt[4];  // per lane
-  int base[5];        // uniform; base[4] = pairs in all
+// order, each sequence's token blocks last first), kept in LDS: per sequence its first pair (the
+// exclusive scan of the pair counts: never decreasing, and a sequence with no pairs shares its
+// successor's), kv_len, q_len and q_start.  In registers they would stay live through every tile's
+// step loop, whose accumulators, queries and fragments fill the file.
+struct CoSeqs {
+  int *off, *kv, *ql, *qs;  // 256 entries each
+  __device__ __forceinline__ explicit CoSeqs(uint8_t* at)
+      : off((int*)at), kv((int*)at + 256), ql((int*)at + 512), qs((int*)at + 768) {}
 };
 
-__device__ __forceinline__ CoPairs co_pairs(const Params& p, const SeqInfo wsi[4], int pf_min, int lane) {
-  CoPairs cp;
+// Fills the tables (wave 0 writes); returns the number of pairs.
+__device__ __forceinline__ int co_pairs(const Params& p, const SeqInfo wsi[4], int pf_min, int lane, int wv,
+                                        const CoSeqs& sq) {
   int base = 0;
 #pragma unroll
   for (int w = 0; w < 4; ++w) {
     const int nt = pf_tiles_of(p, wsi[w], pf_min);
     const int incl = wave_incl_scan32(nt, lane);
-    cp.nt[w] = nt;
-    cp.off[w] = incl - nt;
-    cp.base[w] = base;
+    if (wv == 0) {
+      const int i = 64 * w + lane;
+      sq.off[i] = base + incl - nt;
+      sq.kv[i] = wsi[w].kv_len;
+      sq.ql[i] = wsi[w].q_len;
+      sq.qs[i] = wsi[w].q_start;
+    }
     base += rl(incl, 63);
   }
-  cp.base[4] = base;
-  return cp;
+  return base;
 }
 
-// The tile of pair pi (< base[4]) and kv head h.  Wave-collective.
-__device__ __forceinline__ PfTile co_tile_of(const Params& p, const SeqInfo wsi[4], const CoPairs& cp, int pi, int h) {
+// The tile of pair pi (below the pair count) and kv head h.  Wave-collective.
+__device__ __forceinline__ PfTile co_tile_of(const Params& p, const CoSeqs& sq, int pi, int h, int lane) {
   PfTile tl;
-  tl.seq = -1;
   tl.c_lo = tl.c_hi = 0;
+  // the last sequence whose first pair is <= pi holds it (off[0] = 0, and off never decreases)
+  int seq = -1;
 #pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    if (pi >= cp.base[w] && pi < cp.base[w + 1]) {
-      const int r = pi - cp.base[w];
-      // the last lane whose first pair is <= r holds pair r (offsets never decrease, and a later lane
-      // with no pairs has an offset above r)
-      const int idx = __popcll(__ballot(cp.off[w] <= r)) - 1;
-      const int k = r - rl(cp.off[w], idx), nt = rl(cp.nt[w], idx);
-      tl.seq = 64 * w + idx;
-      tl.kv_len = rl(wsi[w].kv_len, idx);
-      tl.q_len = rl(wsi[w].q_len, idx);
-      tl.q_start = rl(wsi[w].q_start, idx);
-      tl.h = h;
-      tl.tok0 = (nt - 1 - k) * p.pf_tq;  // last token block first
-      tl.ntok = tl.q_len - tl.tok0 < p.pf_tq ? tl.q_len - tl.tok0 : p.pf_tq;
-    }
-  }
-  if (tl.seq >= 0) pf_tile_chunks(p, tl);
+  for (int w = 0; w < 4; ++w) seq += __popcll(__ballot(sq.off[64 * w + lane] <= pi));
+  seq = uni(seq);
+  const int k = pi - uni(sq.off[seq]);
+  tl.seq = seq;
+  tl.kv_len = uni(sq.kv[seq]);
+  tl.q_len = uni(sq.ql[seq]);
+  tl.q_start = uni(sq.qs[seq]);
+  const int nt = (tl.q_len + p.pf_tq - 1) / p.pf_tq;
+  tl.h = h;
+  tl.tok0 = (nt - 1 - k) * p.pf_tq;  // last token block first
+  tl.ntok = tl.q_len - tl.tok0 < p.pf_tq ? tl.q_len - tl.tok0 : p.pf_tq;
+  pf_tile_chunks(p, tl);
   return tl;
 }
 
@@ -2503,9 +2817,10 @@ __device__ __forceinline__ int co_tile_parts(int sz, int np) {
 // workgroup writes every unit's key (one thread per unit: a binary search over the sequences'
 // first pairs finds its sequence), ranks them in LDS and maps queue position r to the unit of rank
 // r / Hkv, kv head r % Hkv.  Calls with more units than kPfOrderMax keep the pair order unsplit.
-template <int MODE>
+template <int MODE, int DT, bool UPG>
 __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], int pf_min, uint8_t* lds, int* s_tile,
-                                        int lane, int wv, int n, int j, int& err, int gpre, bool pf_first) {
+                                        int lane, int wv, int D, int& err, int gpre, bool pf_first) {
+  using L = CoLds<MODE, DT, UPG>;
   RPA_TL(tl_set(TL_TILES0, tl_clock());)
   // fixed first positions when every CU holds a prefill-first workgroup (below): b and b + grid/2
   // share a CU and an XCD (b mod 8), so the pair's positions in that XCD's queue are k and
@@ -2520,8 +2835,8 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
     }
   }
   TlAcc ta;
-  const CoPairs cp = co_pairs(p, wsi, pf_min, lane);
-  const int npairs = cp.base[4];
+  const CoSeqs sqs(lds + L::kSeqs);
+  const int npairs = co_pairs(p, wsi, pf_min, lane, wv, sqs);
   int np = 1;
   if (npairs * p.Hkv < p.grid && npairs * p.Hkv <= p.co_split_max) {
     np = p.grid / (npairs * p.Hkv);
@@ -2532,36 +2847,21 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
   const int nunits = npairs * np;
   const bool ranked = nunits <= kPfOrderMax;
   int nvalid = nunits;
-  int* pkey = (int*)(lds + kCoOrderBase);
+  int* pkey = (int*)(lds + L::kOrder);
   int* pord = pkey + kPfOrderMax;
-  const CoLane cln = co_lane<MODE>(p, wv, lane);
+  CoLoads<MODE, DT, UPG> ld;
+  ld.init(p, D, wv, lane);
+  __syncthreads();
   if (ranked) {
-    // per sequence (256 entries each, over pord's area and the page table until they are
-    // written): its first pair (the exclusive scan of the pair counts: never decreasing, and a
-    // sequence with no pairs shares its successor's), kv_len, q_len
-    int* sq_off = pord;
-    int* sq_kv = pord + 256;
-    int* sq_ql = (int*)(lds + kCoPageBase);
-    static_assert(kCoPages * 12 >= 256 * 4, "sequence table over the page-id and scale tables");
-    if (wv == 0) {
-#pragma unroll
-      for (int w = 0; w < 4; ++w) {
-        const int i = 64 * w + lane;
-        sq_off[i] = cp.base[w] + cp.off[w];
-        sq_kv[i] = wsi[w].kv_len;
-        sq_ql[i] = wsi[w].q_len;
-      }
-    }
-    __syncthreads();
     for (int u = threadIdx.x; u < nunits; u += blockDim.x) {
       const int pair = u / np, part = u - pair * np;
-      int seq = 0;  // the last sequence whose first pair is <= pair (sq_off[0] = 0)
+      int seq = 0;  // the last sequence whose first pair is <= pair (off[0] = 0)
 #pragma unroll
       for (int step = 128; step > 0; step >>= 1)
-        if (sq_off[seq + step] <= pair) seq += step;
-      const int k = pair - sq_off[seq], q_len = sq_ql[seq];
+        if (sqs.off[seq + step] <= pair) seq += step;
+      const int k = pair - sqs.off[seq], q_len = sqs.ql[seq];
       const int nt = (q_len + p.pf_tq - 1) / p.pf_tq;
-      const int sz = co_pair_size(p, sq_kv[seq], q_len, nt, k);
+      const int sz = co_pair_size(p, sqs.kv[seq], q_len, nt, k);
       const int parts = co_tile_parts(sz, np);
       int psz = part < parts ? (sz * (part + 1)) / parts - (sz * part) / parts : -1;
       psz = psz < 0x7fff ? psz : 0x7fff;  // keys stay positive
@@ -2583,7 +2883,8 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
       const int ki = pkey[i];
       if (ki < 0) continue;
       int r = 0;
-      for (int k4 = 0; k4 < n4; ++k4) {
+#pragma unroll 8
+      for (int k4 = 0; k4 < n4; ++k4) {  // (reads of eight in flight)
         const int4 v = ((const int4*)pkey)[k4];
         r += (v.x > ki) + (v.y > ki) + (v.z > ki) + (v.w > ki);
       }
@@ -2657,8 +2958,8 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
       part = u - pair * np;
       unit_np = np;
     }
-    PfTile tl = co_tile_of(p, wsi, cp, pair, h);
-    if (tl.seq < 0 || tl.c_hi <= tl.c_lo) continue;
+    PfTile tl = co_tile_of(p, sqs, pair, h, lane);
+    if (tl.c_hi <= tl.c_lo) continue;
     int slot = -1;
     const int parts = co_tile_parts(tl.c_hi - tl.c_lo, unit_np);
     if (parts > 1) {
@@ -2679,7 +2980,7 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
         d->valid[threadIdx.x] = 1;
       }
     }
-    co_tile<MODE>(p, tl, cln, lds, wv, lane, n, j, err, slot, ta);
+    co_tile<MODE, DT, UPG>(p, tl, ld, lds, wv, lane, err, slot, ta);
   }
   RPA_TL(tl_set(TL_NTILES, ta.tiles); tl_set(TL_NSTEPS, ta.steps); tl_set(TL_QUEUE, ta.queue);
          tl_set(TL_SETUP, ta.setup); tl_set(TL_LOOP, ta.loop); tl_set(TL_WRITE, ta.write);)
@@ -2820,11 +3121,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   }
   const int gd = p.grid - gpre;  // stream-K workgroup count
   RPA_TL(tl_set(TL_SCHED, tl_clock()); int tl_role = pf_first ? 1 : 0;)
-  if (kTiles && pf_first) {
-    if constexpr (CO)
-      co_role<MODE>(p, wsi, pf_min, smem, &s_tile, lane, wv, n, j, err, gpre, pf_first);
-    else if constexpr (MODE == KV_BF16)  // (HG == 8: one K and one V piece per thread per chunk)
-      pf_role<1, UPG>(p, wsi, pf_min, pf_total, smem, &s_tile, lane, wv, n, j, err);
+  if constexpr (kTiles && !CO && MODE == KV_BF16) {  // (HG == 8: one K and one V piece per thread per chunk)
+    if (pf_first) pf_role<1, UPG>(p, wsi, pf_min, pf_total, smem, &s_tile, lane, wv, n, j, err);
   }
   const Partition pt = make_partition_fast(W, gd > 0 ? gd : 1);
   const long long u0 = uni64(range_start(bd, pt)), u1 = uni64(range_start(bd + 1, pt));
@@ -2921,10 +3219,12 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     }
   }
   RPA_TL(tl_set(TL_DEC, tl_clock());)
-  if (CO && !pf_first && pf_total > 0) {
-    __syncthreads();  // every wave is done with its stream-K LDS regions
-    RPA_TL(tl_role |= 4;)
-    co_role<MODE>(p, wsi, pf_min, smem, &s_tile, lane, wv, n, j, err, gpre, pf_first);
+  if constexpr (CO) {
+    if (pf_total > 0) {
+      if (!pf_first) __syncthreads();  // every wave is done with its stream-K LDS regions
+      RPA_TL(if (!pf_first) tl_role |= 4;)
+      co_role<MODE, kD, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, D, err, gpre, pf_first);
+    }
   }
 
   {  // rows at or past cu_q_lens[num_seqs] belong to no sequence: zero them
@@ -4598,8 +4898,11 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     return fail(RPA_E_HIP, "hipEventRecord(begin) failed");
   const bool upg = p.S % KV_CHUNK == 0;
   const dim3 grid(p.grid), block(64 * p.HG);
-  const size_t lds = (size_t)p.HG * (kVtBytes + (mode == KV_BF16_FUSED ? kRelStage : 0) +
-                                     (p.D > kD ? kWideSlot : 0));
+  size_t lds = (size_t)p.HG * (kVtBytes + (mode == KV_BF16_FUSED ? kRelStage : 0) + (p.D > kD ? kWideSlot : 0));
+  if (p.co) {
+    const size_t tiles = mode == KV_FP8 ? CoLds<KV_FP8, kD, true>::kBytes : CoLds<KV_BF16, kD, true>::kBytes;
+    lds = lds > tiles ? lds : tiles;
+  }
   if (mode == KV_BF16_FUSED) {
     if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_FUSED, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_FUSED, false>), grid, block, lds, st, p);
