@@ -69,16 +69,19 @@ typedef struct rpa_shape {
  *                  workgroups, at least one (with 8-wave workgroups, 4 is one
  *                  workgroup per two CUs); 0 or 8: the kernel's occupancy, 8
  *                  waves per CU (rpa_attention_grid reports the result);
- *   prefill_tiles  sequences with at least 16 query tokens (bf16 KV without
- *                  scales, the default mask value): 2 = the attention kernel's
- *                  own MFMA prefill tiles, in two 4-wave workgroups per CU (one
- *                  prefill, one stream-K) when the page size is a multiple of
- *                  32, Hkv a multiple of 4 and num_tokens >= max_num_seqs + 15,
- *                  else in one 8-wave workgroup per CU (8 kv heads per
- *                  workgroup); 3 = those tiles in one 8-wave workgroup per CU;
- *                  1 = the standalone prefill kernel (page size a multiple of
- *                  64); 0 = 2, else 1, whichever applies first; -1 = causal row
- *                  blocks of the stream-K role (also whenever none applies);
+ *   prefill_tiles  sequences with at least 16 query tokens: 2 = the attention
+ *                  kernel's own MFMA prefill tiles (num_tokens >= max_num_seqs +
+ *                  15), in two 4-wave workgroups per CU (one prefill, one
+ *                  stream-K): head_dim 128 with bf16 KV (scalar scales included:
+ *                  page size a multiple of 32, Hkv a multiple of 4) or fp8 KV,
+ *                  head_dim 64 with plain bf16 or fp8 KV; plain bf16 KV with the
+ *                  default mask value, Hkv a multiple of 8 and another page size:
+ *                  in one 8-wave workgroup per CU; 3 = the tiles in one 8-wave
+ *                  workgroup per CU (plain bf16 KV, default mask value, Hkv a
+ *                  multiple of 8); 1 = the standalone prefill kernel (page size a
+ *                  multiple of 64); 0 = 2, else 1, whichever applies first; -1 =
+ *                  causal row blocks of the stream-K role (also whenever none
+ *                  applies);
  *   prefill_cost   > 0: the cost of one prefill-tile chunk step in stream-K
  *                  units, which sets the work split between the two roles
  *                  (0 = 0.45). */

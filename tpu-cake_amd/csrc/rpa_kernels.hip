@@ -208,6 +208,9 @@ struct Params {
   // share a CU); the prefill tiles are 128 rows, one prefill workgroup beside one stream-K
   // workgroup on a CU, and stream-K workgroups join the tile queue when their range is done
   int co;
+  int SUB;                     // stream-K workers per workgroup: 4 / HG in the co-resident layout, else 1
+  int lockstep;                // the workgroup's waves walk one worker's units together
+  int dgrid;                   // stream-K workers of the grid (grid * SUB): the split descriptors' count
   int co_split_max;            // split co tiles the workspace holds
   struct CoDesc* co_desc;      // [co_split_max]
   int pk_grid;                 // prefill-kernel workgroups
@@ -1176,7 +1179,7 @@ __device__ __forceinline__ void write_split_desc(const Params& p, const Cursor& 
   }
 }
 
-template <int MODE, bool UPG>
+template <int MODE, bool UPG, bool CO>
 __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n, int j, int b, long long u,
                                      long long u0, long long u1, Window& win, Cursor& cur, Cursor& nxt,
                                      Pages& pg_nxt, const HalfRegs<MODE>& k_cur, const HalfRegs<MODE>& v_cur,
@@ -1193,8 +1196,8 @@ __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n,
   const Pages pg_ahead = load_pages<MODE, UPG>(p, ahead, n);
   const UnitAddr nx_addr = unit_addr(p, nxt, pg_nxt, n, j, wv, err, D);
   // keep the workgroup's waves (the kv heads of one group) in step, so the heads' slices of the
-  // same keys reach the memory system together
-  __syncthreads();
+  // same keys reach the memory system together (a workgroup of several workers has nothing to keep)
+  if (!CO || p.lockstep) __syncthreads();
   load_half<MODE, UPG>(p, nx_addr, 0, k_nxt, D);
 
   if (u == u0 || cur.c == 0) begin_row_block(p, cur, st, n);
@@ -1475,7 +1478,7 @@ __device__ __forceinline__ void compute_unit_line(const Params& p, const Cursor&
   __builtin_amdgcn_sched_group_barrier(0x008, 8, 0);
 }
 
-template <int MODE, bool UPG, int DN = 0>
+template <int MODE, bool UPG, int DN, bool CO>
 __device__ __forceinline__ void step_line(const Params& p, int nseq, int lane, int n, int j, int b, long long u,
                                           long long u0, long long u1, Window& win, Cursor& cur, Cursor& nxt,
                                           Pages& pg_nxt, LineRegs& k, LineRegs& v, f32x4 bias[2], bf16x8 q[4],
@@ -1489,7 +1492,7 @@ __device__ __forceinline__ void step_line(const Params& p, int nseq, int lane, i
     ahead.nch = 0;
   const Pages pg_ahead = load_pages<MODE, UPG>(p, ahead, n);
   const LineAddr nx_addr = line_addr<MODE, UPG, DN>(p, nxt, pg_nxt, lane, n, j, wv, err, D);
-  __syncthreads();
+  if (!CO || p.lockstep) __syncthreads();
   load_lines<MODE, UPG, DN>(p, nx_addr, lane, 0, k, D);  // the next unit's K (this unit's K is in the tile)
   LineBias bias_nx;
   load_line_bias<MODE>(p, nxt, nx_addr, lane, n, j, wv, bias_nx);
@@ -2989,14 +2992,17 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
 // CO: the co-resident layout's instantiation (p.co set), with the co-resident prefill role; the
 // other instantiations carry the 8-wave prefill role (plain bf16 KV) or none, so the decode-only
 // launches keep the registers of a kernel without the co-resident role.
-// NW: a narrow head dim (p.D < kD; decode role only, every row through stream-K).  DN: a narrow
+// DT: the co-resident tiles' head dim (64 or 128).  NW: a narrow head dim (p.D < kD; without CO decode role
+// only, every row through stream-K).  DN: a narrow
 // head dim of 32 or 64 fixed at compile time, whose full-line loads read whole DN-element rows
 // (Lines<DN>).
-template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0>
+template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rpa_attn_kernel(Params p) {
   static_assert(DN == 0 || (NW && UPG && (DN == 32 || DN == 64)), "DN: a narrow instantiation of 32 or 64");
-  constexpr bool kTiles = NW ? false : CO ? co_tiles<MODE>() : MODE == KV_BF16;  // a prefill-tile role exists
-  const int D = DN ? DN : NW ? p.D : kD;
+  static_assert(!CO || co_tiles<MODE>(), "CO: a mode with co-resident tiles");
+  static_assert(!(CO && NW) || DT == 64, "a narrow co-resident instantiation: 64-dim heads");
+  constexpr bool kTiles = CO ? true : NW ? false : MODE == KV_BF16;  // a prefill-tile role exists
+  const int D = DN ? DN : CO ? DT : NW ? p.D : kD;
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];  // HG x (V region, K tile)
   const int lane = threadIdx.x & 63;
   const int wv = uni(threadIdx.x >> 6);
@@ -3119,7 +3125,15 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     pf_first = b < gpre;
     bd = b - gpre;
   }
-  const int gd = p.grid - gpre;  // stream-K workgroup count
+  int gd = p.grid - gpre;  // stream-K workgroup count
+  // a co-resident workgroup's four waves are SUB stream-K workers of HG waves (HG 3: one wave idles)
+  int wh = wv;  // this wave's kv head of its worker's group
+  if constexpr (CO) {
+    const int sub = uni(wv / p.HG);
+    wh = wv - sub * p.HG;
+    bd = bd >= 0 && sub < p.SUB ? bd * p.SUB + sub : -1;
+    gd *= p.SUB;
+  }
   RPA_TL(tl_set(TL_SCHED, tl_clock()); int tl_role = pf_first ? 1 : 0;)
   if constexpr (kTiles && !CO && MODE == KV_BF16) {  // (HG == 8: one K and one V piece per thread per chunk)
     if (pf_first) pf_role<1, UPG>(p, wsi, pf_min, pf_total, smem, &s_tile, lane, wv, n, j, err);
@@ -3178,10 +3192,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         // K, bias, queries, V: the loop's order (vmcnt retires in order, and the compiler
         // counts each wait for the least favourable path into it, this prologue included)
         {
-          const LineAddr a0 = line_addr<MODE, UPG, DN>(p, cur, pg_cur, lane, n, j, wv, err, D);
+          const LineAddr a0 = line_addr<MODE, UPG, DN>(p, cur, pg_cur, lane, n, j, wh, err, D);
           load_lines<MODE, UPG, DN>(p, a0, lane, 0, k, D);
-          load_line_bias<MODE>(p, cur, a0, lane, n, j, wv, bias_in);
-          load_q<MODE>(p, cur, n, j, wv, q, rst, MODE == KV_BF16_FUSED ? p.D : D);
+          load_line_bias<MODE>(p, cur, a0, lane, n, j, wh, bias_in);
+          load_q<MODE>(p, cur, n, j, wh, q, rst, MODE == KV_BF16_FUSED ? p.D : D);
           load_lines<MODE, UPG, DN>(p, a0, lane, 1, v, D);
         }
         RPA_TL(tl_set(TL_FIRST, tl_clock()); tl_set(TL_UNITS, u1 - u0); tl_role |= 2;)
@@ -3190,17 +3204,17 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         RowState st;
         long long u = u0;
         for (;;) {
-          step_line<MODE, UPG, DN>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, k, v, bias, q, rst, st, vt,
-                               kt, rs, err, pt, wv, D);
+          step_line<MODE, UPG, DN, CO>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, k, v, bias, q, rst, st, vt,
+                               kt, rs, err, pt, wh, D);
           if (++u >= u1) break;
         }
       } else {
         HalfRegs<MODE> ka, va, kb, vb;
         bf16x8 q[4];
         {  // K, queries, V: the loop's order (as above)
-          const UnitAddr a0 = unit_addr(p, cur, pg_cur, n, j, wv, err, D);
+          const UnitAddr a0 = unit_addr(p, cur, pg_cur, n, j, wh, err, D);
           load_half<MODE, UPG>(p, a0, 0, ka, D);
-          load_q<MODE>(p, cur, n, j, wv, q, nullptr, D);
+          load_q<MODE>(p, cur, n, j, wh, q, nullptr, D);
           load_half<MODE, UPG>(p, a0, 1, va, D);
         }
         RPA_TL(tl_set(TL_FIRST, tl_clock()); tl_set(TL_UNITS, u1 - u0); tl_role |= 2;)
@@ -3208,11 +3222,11 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
 
         long long u = u0;
         for (;;) {
-          step<MODE, UPG>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, ka, va, kb, vb, q, st, vt, err, pt,
-                          wv, D);
+          step<MODE, UPG, CO>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, ka, va, kb, vb, q, st, vt, err, pt,
+                          wh, D);
           if (++u >= u1) break;
-          step<MODE, UPG>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, kb, vb, ka, va, q, st, vt, err, pt,
-                          wv, D);
+          step<MODE, UPG, CO>(p, nseq, lane, n, j, bd, u, u0, u1, win, cur, nxt, pg_nxt, kb, vb, ka, va, q, st, vt, err, pt,
+                          wh, D);
           if (++u >= u1) break;
         }
       }
@@ -3223,7 +3237,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (pf_total > 0) {
       if (!pf_first) __syncthreads();  // every wave is done with its stream-K LDS regions
       RPA_TL(if (!pf_first) tl_role |= 4;)
-      co_role<MODE, kD, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, D, err, gpre, pf_first);
+      co_role<MODE, DT, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, D, err, gpre, pf_first);
     }
   }
 
@@ -3870,7 +3884,7 @@ __device__ __forceinline__ void combine_heavy(const Params& p, int hb, float (*r
   SplitDesc d = p.heavy_desc[slot];
   asm volatile("" : "+v"(f), "+v"(d.q_start), "+v"(d.q_len), "+v"(d.h), "+v"(d.rb), "+v"(d.b0));
   f = __builtin_amdgcn_readfirstlane(f);
-  if (f <= 0 || f > p.grid) return;
+  if (f <= 0 || f > p.dgrid) return;
   const int b = f - 1;
   const int t = threadIdx.x, wv = t >> 6, lane = t & 63;
   const int ncontrib = (int)(b - d.b0 + 1), nrows = rows_of(p, d);
@@ -3977,6 +3991,7 @@ __device__ __forceinline__ void combine_co_split(const Params& p, int idx) {
 #pragma unroll 1
   for (int row = 32 * g + (t >> 3); row < 32 * g + 32; row += (int)(blockDim.x >> 3)) {
     if (row >= d.ntok * p.G) break;
+    if (c16 >= p.D) continue;  // (64-dim rows)
     f32x4 o[4];
     float m = -INFINITY, l = 0.f;
 #pragma unroll
@@ -3994,7 +4009,7 @@ __device__ __forceinline__ void combine_co_split(const Params& p, int idx) {
     }
     const float inv = 1.f / l;
     const int tok = row / p.G, head = d.h * p.G + (row - tok * p.G);
-    uint16_t* op = p.out + ((size_t)(d.q_row0 + tok) * p.Hq + head) * kD + c16;
+    uint16_t* op = p.out + ((size_t)(d.q_row0 + tok) * p.Hq + head) * p.D + c16;
     u32x4 w0, w1;
     w0[0] = pack_bf16x2(o[0][0] * inv, o[0][1] * inv);
     w0[1] = pack_bf16x2(o[0][2] * inv, o[0][3] * inv);
@@ -4021,14 +4036,14 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
   if (blockIdx.x == 0 && threadIdx.x < kXcds) p.err[kQueueWord + threadIdx.x] = 0;  // tile queues, for the next call
   // the heavy-merge helpers first (a heavy merge is the longest, so it starts with the launch),
   // then the (descriptor, head) merges, then the rest
-  const int nheavy = heavy_slots(p.grid) * p.HG * kHeavySlices;
+  const int nheavy = heavy_slots(p.dgrid) * p.HG * kHeavySlices;
   if ((int)blockIdx.x < nheavy) {
     combine_heavy<CW>(p, blockIdx.x, red, redml);
     return;
   }
   const int mb = (int)blockIdx.x - nheavy;
-  if (mb >= p.grid * p.HG) {
-    const int hb = mb - p.grid * p.HG;
+  if (mb >= p.dgrid * p.HG) {
+    const int hb = mb - p.dgrid * p.HG;
     if (p.fused)
       fused_store_token(p, hb);
     else if (p.co)
@@ -4038,7 +4053,7 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
     return;
   }
   // descriptor (last first: long splits end in late workgroups), wave (head) of its group
-  const int bi = mb / p.HG, hw = mb - bi * p.HG, b = p.grid - 1 - bi;
+  const int bi = mb / p.HG, hw = mb - bi * p.HG, b = p.dgrid - 1 - bi;
   // the flag and the fields in one round trip (the empty asm keeps the compiler from moving the
   // field loads behind the flag test)
   int valid = p.desc[b].valid[hw];
@@ -4482,6 +4497,8 @@ Params base_params(const rpa_shape_t* s) {
     p.HG = 2 * g;
   }
   p.NG = (p.D == 2 * kD ? 2 * p.Hkv : p.Hkv) / p.HG;
+  p.SUB = 1;
+  p.lockstep = 1;
   return p;
 }
 
@@ -4754,31 +4771,46 @@ int nominal_per_cu(int hg, size_t lds) {
 }
 
 // Where the rows of sequences with >= 16 query tokens go, and the workgroup shape that follows:
-//   prefill_tiles 2 or 0, bf16 KV (plain or with scalar k/v scales) or fp8 KV, any mask value,
-//     page size a multiple of 32, Hkv a multiple of 4, and num_tokens >= max_num_seqs + 15 (the
-//     batch can hold such a sequence; a batch of one token per sequence keeps the decode layout):
-//     the attention kernel's tiles in the co-resident layout (4-wave workgroups, two per CU, one
-//     prefill and one stream-K workgroup side by side);
+//   prefill_tiles 2 or 0 and num_tokens >= max_num_seqs + 15 (the batch can hold such a sequence; a batch of
+//     one token per sequence keeps the decode layout), any mask value, kv_pages 16-byte aligned (the tiles'
+//     LDS DMA): the attention kernel's tiles in the co-resident layout (4-wave workgroups, two per CU, one
+//     prefill and one stream-K workgroup side by side), for
+//       128-dim heads, bf16 KV (plain or with scalar k/v scales) or fp8 KV, page size a multiple of 32, Hkv
+//       a multiple of 4: a workgroup is one stream-K worker of four kv heads;
+//       128- or 64-dim heads, plain bf16 or fp8 KV, any other page size or kv head count: a workgroup holds
+//       4 / HG workers -- except where the 8-wave layout below takes plain bf16 pools.  As 16-row stream-K
+//       blocks those rows read K and V again for every 16 of them: a page-16 chunked prefill (5 chunks of up
+//       to 1023 tokens, Hq 8 / Hkv 2) took 145 us a call against 59 in tiles, a 64-dim mixed batch (24
+//       decode rows, 4 chunks of 512, Hq 32 / Hkv 8) 353 against 78;
 //   prefill_tiles 3, or 2 / 0 otherwise, for plain bf16 KV whose masked keys get weight 0 and
 //     eight kv heads per workgroup: the attention kernel's tiles in 8-wave workgroups, one per
 //     CU, roles split by CU;
 //   prefill_tiles 1, or 0 when none of these applies: the prefill kernel (plain bf16 KV, masked
 //     keys at weight 0, chunks in one page: page size a multiple of 64);
 //   otherwise, and with -1: causal row blocks of the stream-K role.
-void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_options_t* opt) {
-  if (p.D != kD) return;  // a narrow head dim: every row through stream-K
+void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_options_t* opt, bool aligned) {
   const int pt = opt->prefill_tiles;
   const bool bf = mode == KV_BF16 && p.skip_masked;
+  const bool tiles_ok = p.D == kD && bf && p.HG == 8 && p.G <= 32 * p.HG;
   const bool co_mode = mode == KV_BF16 || mode == KV_BF16_SCALED || mode == KV_FP8;  // any mask value
-  const bool co_ok = co_mode && (pt == 0 || pt == 2) && p.S % KV_CHUNK == 0 && p.Hkv % kCoWaves == 0 &&
-                     p.G <= 32 * kCoWaves && (long long)shape->num_tokens >= (long long)shape->max_num_seqs + 15;
-  const bool tiles_ok = bf && p.HG == 8 && p.G <= 32 * p.HG;
+  const bool co_may = co_mode && aligned && (pt == 0 || pt == 2);
+  const bool co_one = co_may && p.D == kD && p.S % KV_CHUNK == 0 && p.Hkv % kCoWaves == 0 &&
+                      p.G <= 32 * kCoWaves && (long long)shape->num_tokens >= (long long)shape->max_num_seqs + 15;
+  const bool co_any = co_may && (p.D == kD || p.D == 64) && mode != KV_BF16_SCALED && !tiles_ok &&
+                      p.G <= 32 * kCoWaves &&
+                      (p.S % KV_CHUNK == 0 || (unsigned long long)p.P * p.S <= 0xffffffffull) &&  // 32-bit pool rows
+                      (long long)shape->num_tokens >= (long long)shape->max_num_seqs + 15;
+  const bool co_ok = co_one || co_any;
+  if (p.D != kD && !co_ok) return;  // another head dim: every row through stream-K
   const bool pk_ok = bf && p.G <= kPkRows && p.S % kPkChunk == 0;
   const float cost = opt->prefill_cost > 0.f ? opt->prefill_cost : kPfCost;
   if (co_ok) {
     p.co = 1;
-    p.HG = kCoWaves;
-    p.NG = p.Hkv / kCoWaves;
+    p.HG = p.Hkv < kCoWaves ? p.Hkv : kCoWaves;  // the largest divisor of Hkv that is <= 4
+    while (p.Hkv % p.HG) --p.HG;
+    p.NG = p.Hkv / p.HG;
+    p.SUB = kCoWaves / p.HG;
+    p.lockstep = p.HG == kCoWaves;
     p.pf_tq = 32 * kCoWaves / p.G;
     p.pf_min = 16;
     p.pf_cost = cost;
@@ -4792,6 +4824,19 @@ void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_opt
     p.pf_cost = cost;
   }
 }
+
+// LDS of a co-resident workgroup's tile role.
+size_t co_lds_bytes(int mode, bool upg, int D) {
+  const bool fp8 = mode == KV_FP8;
+  if (D == 64)
+    return fp8 ? (upg ? CoLds<KV_FP8, 64, true>::kBytes : CoLds<KV_FP8, 64, false>::kBytes)
+               : (upg ? CoLds<KV_BF16, 64, true>::kBytes : CoLds<KV_BF16, 64, false>::kBytes);
+  return fp8 ? (upg ? CoLds<KV_FP8, kD, true>::kBytes : CoLds<KV_FP8, kD, false>::kBytes)
+             : (upg ? CoLds<KV_BF16, kD, true>::kBytes : CoLds<KV_BF16, kD, false>::kBytes);
+}
+static_assert(CoLds<KV_FP8, kD, false>::kBytes + 64 <= 80 * 1024 && CoLds<KV_BF16, kD, false>::kBytes + 64 <= 80 * 1024 &&
+                  CoLds<KV_FP8, kD, true>::kBytes + 64 <= 80 * 1024 && CoLds<KV_BF16, kD, true>::kBytes + 64 <= 80 * 1024,
+              "two co-resident workgroups per CU");
 
 static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const void* q, const void* kv_pages,
                       const float* kv_scales, const int32_t* kv_lens, const int32_t* page_indices,
@@ -4883,8 +4928,10 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     if (kv_scales) return fail(RPA_E_INVALID, "kv_scales is only used with fp8 kv_pages");
     if (opt->has_k_scale || opt->has_v_scale) mode = KV_BF16_SCALED;
   }
-  resolve_layout(p, mode, shape, opt);
-  p.grid = grid_for_call(d, mode, p.HG, opt->waves_per_cu);
+  resolve_layout(p, mode, shape, opt, (uintptr_t)kv_pages % 16 == 0);
+  const int waves = p.co ? kCoWaves : p.HG;  // per workgroup
+  p.grid = grid_for_call(d, mode, waves, opt->waves_per_cu);
+  p.dgrid = p.grid * p.SUB;
   if (p.pf_kernel) p.pk_grid = d.cus;
   // split co tiles: descriptors over the prefill-kernel descriptor area (one PkDesc per CU), partial
   // slots of 128 rows over its partial areas (2 x 256 rows per CU)
@@ -4897,10 +4944,11 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   if (ev_begin && hipEventRecord((hipEvent_t)ev_begin, st) != hipSuccess)
     return fail(RPA_E_HIP, "hipEventRecord(begin) failed");
   const bool upg = p.S % KV_CHUNK == 0;
-  const dim3 grid(p.grid), block(64 * p.HG);
+  const dim3 grid(p.grid), block(64 * waves);
   size_t lds = (size_t)p.HG * (kVtBytes + (mode == KV_BF16_FUSED ? kRelStage : 0) + (p.D > kD ? kWideSlot : 0));
   if (p.co) {
-    const size_t tiles = mode == KV_FP8 ? CoLds<KV_FP8, kD, true>::kBytes : CoLds<KV_BF16, kD, true>::kBytes;
+    const size_t tiles = co_lds_bytes(mode, upg, p.D);
+    lds = (size_t)kCoWaves * kVtBytes;
     lds = lds > tiles ? lds : tiles;
   }
   if (mode == KV_BF16_FUSED) {
@@ -4909,7 +4957,15 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   } else if (mode == KV_BF16_BIAS) {
     if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_BIAS, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_BIAS, false>), grid, block, lds, st, p);
-  } else if (p.D != kD) {  // a narrow head dim (decode role only)
+  } else if (p.co && p.D == 64) {  // 64-dim heads with prefill tiles
+    if (mode == KV_FP8) {
+      if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, true, true, true, 0, 64>), grid, block, lds, st, p);
+      else hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, false, true, true, 0, 64>), grid, block, lds, st, p);
+    } else {
+      if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true, true, 64, 64>), grid, block, lds, st, p);
+      else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true, true, 0, 64>), grid, block, lds, st, p);
+    }
+  } else if (p.D != kD) {  // another head dim (decode role only)
     if (mode == KV_FP8) {
       if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, true, false, true>), grid, block, lds, st, p);
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, false, false, true>), grid, block, lds, st, p);
@@ -4926,7 +4982,8 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true>), grid, block, lds, st, p);
     }
   } else if (mode == KV_FP8) {
-    if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, true, true>), grid, block, lds, st, p);
+    if (p.co && upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, true, true>), grid, block, lds, st, p);
+    else if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, false, true>), grid, block, lds, st, p);
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, false>), grid, block, lds, st, p);
   } else if (mode == KV_BF16_SCALED) {
@@ -4934,7 +4991,8 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false>), grid, block, lds, st, p);
   } else {
-    if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true>), grid, block, lds, st, p);
+    if (p.co && upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true>), grid, block, lds, st, p);
+    else if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true>), grid, block, lds, st, p);
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false>), grid, block, lds, st, p);
   }
@@ -4954,7 +5012,7 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   // the heavy-merge helpers of every slot, then one workgroup per (descriptor, head), then 16 per
   // prefill workgroup; two-wave workgroups when a decode row block has at most 4 rows (G <= 4,
   // no prefill-kernel split tiles), four-wave ones otherwise
-  const dim3 cgrid(p.grid * p.HG + heavy_slots(p.grid) * p.HG * kHeavySlices + (p.pf_kernel ? 16 * p.pk_grid : 0) +
+  const dim3 cgrid(p.dgrid * p.HG + heavy_slots(p.dgrid) * p.HG * kHeavySlices + (p.pf_kernel ? 16 * p.pk_grid : 0) +
                    (p.fused ? p.fused_nseq : 0) + (p.co ? 4 * p.co_split_max : 0));
   if (combine_waves(p) == 2)
     hipLaunchKernelGGL(rpa_combine_kernel<2>, cgrid, dim3(128), 0, st, p);
@@ -4984,19 +5042,20 @@ int rpa_attention_grid(const rpa_shape_t* shape, const rpa_options_t* opt, int32
     mode = KV_FP8;
   else if (opt->has_k_scale || opt->has_v_scale)
     mode = KV_BF16_SCALED;
-  resolve_layout(p, mode, shape, opt);
+  resolve_layout(p, mode, shape, opt, true);
+  const int waves = p.co ? kCoWaves : p.HG;
   int occ;
   if (cus > 0) {
-    occ = cus * nominal_per_cu(p.HG, (size_t)p.HG * kVtBytes);
+    occ = cus * nominal_per_cu(waves, (size_t)waves * kVtBytes);
   } else {
     DeviceInfo d;
     rc = device_info(d);
     if (rc) return rc;
     cus = d.cus;
-    occ = d.grid[mode][p.HG];
+    occ = d.grid[mode][waves];
   }
-  *grid = grid_rule(occ, cus, p.HG, opt->waves_per_cu);
-  *waves_per_workgroup = p.HG;
+  *grid = grid_rule(occ, cus, waves, opt->waves_per_cu);
+  *waves_per_workgroup = waves;
   return RPA_OK;
 }
 
