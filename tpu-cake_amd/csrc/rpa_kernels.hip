@@ -4082,6 +4082,468 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
 }
 
 // ---------------------------------------------------------------------------------------------
+// small calls in one launch: one workgroup per (sequence, kv head)
+// ---------------------------------------------------------------------------------------------
+// A call with at most one query token per sequence slot, short page tables and few (sequence, kv head)
+// pairs is bound by launches and round trips, not by bytes: split over the whole grid it needs a second
+// launch to merge the splits (4.5 us).  Here the eight waves of a workgroup take a sequence's 32-key chunks
+// in turn (wave w: chunks w, w + 8, ...) and merge their (m, l, acc) through LDS.  Two memory round trips:
+// the metadata and the page ids of the wave's first chunks come together (an entry past the sequence's own
+// pages is read, checked and not used), then queries, K and V.
+//
+// The same kernel runs the fused decode step (new token, relative bias, cache write: there is no merge
+// launch to store the token) and the v1 contract (separate caches, bias by key position) over its own
+// caches.  DW: row width computed, 64, 128 or 256 (dims past the real D are zero in Q and not stored).
+//
+// Per call in a captured step, 4 sequences, Hq 8 / Hkv 2, page 16, D 128 (before: split and merged): 32 keys
+// 7.9 -> 4.3 us, 128 keys 10.0 -> 5.2, 512 keys 11.1 -> 8.8; 32 sequences of 512 keys at Hq 32 / Hkv 8
+// 26.1 -> 17.9.  The rule's bounds (direct_call): one CU reads a pair's K and V, so past kDirectElems
+// elements of K the split form is ahead (bf16, D 128, lengths uniform up to the table's end: 1024 keys 1.2 to
+// 1.5x faster here, 2048 keys 0.83 to 1.25x; D 64 still 1.4 to 2.2x at 2048, D 256 0.8 to 1.1x at 1024), and
+// past kDirectGroups pairs the grid is full either way (1024 pairs: bf16 1.07x, fp8 0.8x).
+constexpr int kDirectWaves = 8;
+constexpr int kDirectElems = 1024 * 128;  // keys of a page table x row width
+constexpr int kDirectGroups = 512;        // sequence slots x kv heads: two workgroups per CU
+constexpr int kDirectMaxKeys = 4096;      // (pmagic's range)
+
+struct DirectArgs {
+  const uint8_t* kb;   // K of kv head 0 of pool row 0
+  const uint8_t* vb;   // V of kv head 0 of pool row 0
+  long long row;       // bytes between pool rows (keys)
+  int head;            // bytes between kv heads
+  const uint16_t* bias;  // v1: [Hq, bias_len] by key position
+  int bias_len;
+  uint32_t pmagic;       // ceil(2^31 / S): page_of below 4096 keys is one multiplication
+};
+
+// K or V of a chunk as it comes from memory, whole rows per load: load i covers keys kKeys i ..
+// + kKeys - 1, lane L holding key kKeys i + L / kLanes, 16 bytes at 16 (L % kLanes) of its row.  (Loads
+// in the MFMA operand layout touch 64 bytes of 16 rows each: a probe of one workgroup's reads from L2 ran
+// at 36 bytes/ns per CU that way against 119 with whole rows.)
+template <int MODE, int DW>
+struct DirectHalf {
+  static constexpr int kRow = MODE == KV_FP8 ? DW : 2 * DW;  // bytes of a row as computed
+  static constexpr int kLanes = kRow / 16, kKeys = 64 / kLanes, kLoads = KV_CHUNK / kKeys;
+  u32x4 w[kLoads];
+};
+
+// One chunk of one wave.
+template <int MODE, int DW>
+struct DirectChunk {
+  DirectHalf<MODE, DW> k, v;
+  f32x2 scale;         // fp8: K and V scale of key lane % 32
+  uint16_t b[2][4];    // v1: bias of keys 16 blk + 4j + r; fused: rel_proj[4j + t] at the distance of key 16 blk + n
+};
+
+// A chunk's K or V to bf16 key rows in the wave's region.
+template <int MODE, int DW, int ROW>
+__device__ __forceinline__ void direct_store(uint8_t* vt, const DirectHalf<MODE, DW>& r, int lane, float sc, bool exact) {
+  using H = DirectHalf<MODE, DW>;
+#pragma unroll
+  for (int i = 0; i < H::kLoads; ++i) {
+    const int key = H::kKeys * i + lane / H::kLanes;
+    uint8_t* at = vt + key * ROW + (MODE == KV_FP8 ? 32 : 16) * (lane % H::kLanes);
+    if constexpr (MODE == KV_FP8) {
+      // the key's scale is with lane `key`
+      const float s = __builtin_bit_cast(float, __builtin_amdgcn_ds_bpermute(4 * key, __builtin_bit_cast(int, sc)));
+      const u32x2 lo = {r.w[i][0], r.w[i][1]}, hi = {r.w[i][2], r.w[i][3]};
+      *(u32x4*)at = exact ? fp8x8_to_bf16x8_exact(lo) : fp8x8_to_bf16x8(lo, s);
+      *(u32x4*)(at + 16) = exact ? fp8x8_to_bf16x8_exact(hi) : fp8x8_to_bf16x8(hi, s);
+    } else if constexpr (MODE == KV_BF16_SCALED) {
+      *(u32x4*)at = scale_bf16x8(r.w[i], sc);
+    } else {
+      *(u32x4*)at = r.w[i];
+    }
+  }
+}
+
+// MODE KV_BF16_BIAS: the v1 contract.
+template <int MODE, int DW>
+__global__ __launch_bounds__(64 * kDirectWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void
+rpa_attn_kernel_direct(Params p, DirectArgs a) {
+  constexpr int KS = DW / 32, DB = DW / 16;
+  constexpr int kRowV = 2 * DW + 32;                 // V region: 32 key rows (conflict-free transposing reads)
+  constexpr int kRegion = KV_CHUNK * kRowV;          // ... and, after the chunks, 16 rows of DW + 4 floats
+  constexpr int kRowO = DW + 4;
+  static_assert(16 * kRowO * 4 <= kRegion, "a wave's accumulators fit its V region");
+  constexpr int kElem = MODE == KV_FP8 ? 1 : 2;
+  constexpr bool kFused = MODE == KV_BF16_FUSED;
+  constexpr bool kPrefetch = DW <= 128;  // (two chunks of 256-dim rows do not fit the registers)
+  extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
+  float* sml = (float*)(smem + kDirectWaves * kRegion);  // [wave][row][m, l]
+  const int lane = threadIdx.x & 63, wv = uni(threadIdx.x >> 6);
+  const int n = lane & 15, j = lane >> 4;
+  uint8_t* vt = smem + wv * kRegion;
+  const int i = blockIdx.x / p.Hkv, h = blockIdx.x - i * p.Hkv;
+  const int D = p.D;
+  int err = 0;
+
+  // round trip 1: metadata, page ids of the wave's chunks in [0, kDirectKeys)
+  const long long cap = (long long)p.PPS * p.S;
+  bool store = true;  // fused: the new token's slot exists
+  constexpr bool kV1 = MODE == KV_BF16_BIAS;  // one query token per sequence, no cu_q_lens
+  const int ns_raw = kFused || kV1 ? p.fused_nseq : p.num_seqs[0];
+  int kv = p.kv_lens[i];
+  const int c0 = kFused || kV1 ? i : p.cu_q_lens[i];
+  const int c1 = kV1 ? i + 1 : kFused ? p.cu_kv[i] : p.cu_q_lens[i + 1];
+  size_t prow = (size_t)i * p.PPS;
+  auto page = [&](int kt) { return (int)__umulhi((unsigned)kt << 1, a.pmagic); };
+  auto load_ids = [&](int c) {  // page id of key lane % 32 of chunk c (past the table: its last entry)
+    int kt = c * KV_CHUNK + (lane & 31);
+    kt = kt < cap ? kt : (int)cap - 1;
+    size_t at = prow + page(kt);
+    if (kFused) at = at < (size_t)p.fused_entries ? at : 0;
+    return p.page_indices[at];
+  };
+  int id0 = 0, id1 = 0;  // of chunks wv and wv + kDirectWaves
+  if constexpr (!kFused) {
+    id0 = load_ids(wv);
+    id1 = load_ids(wv + kDirectWaves);
+  }
+  int nseq = uni(ns_raw);
+  nseq = nseq < 0 ? 0 : (nseq > p.Nmax ? p.Nmax : nseq);
+  kv = uni(kv);
+  const int q0 = uni(c0);
+  int ql = kFused ? 1 : uni(c1) - q0;
+  bool live = i < nseq;
+  if (kv > cap) {
+    if (live) err |= kFused ? ERR_KVLEN | ERR_PAGE : ERR_KVLEN;
+    kv = (int)cap;
+    store = false;
+  }
+  kv = kv < 0 ? 0 : kv;
+  if (!kFused && (q0 < 0 || ql < 0 || uni(c1) > p.T)) {
+    if (live) err |= ERR_QROW;
+    ql = 0;
+  }
+  if (live && ql > kv) err |= ERR_QLEN;
+  if constexpr (kFused) {  // (make_fused_seq) the sequence's pages start at entry cu_kv / S
+    const int cu = uni(c1), pb = page_of(cu, p), npg = kv > 0 ? page(kv - 1) + 1 : 0;
+    if (cu < 0 || pb * p.S != cu || (long long)pb + npg > (long long)p.fused_entries) {
+      if (live) err |= ERR_PAGE;
+      live = false;
+    }
+    prow = live ? pb : 0;
+    id0 = load_ids(wv);
+    id1 = load_ids(wv + kDirectWaves);
+  }
+  live = live && ql > 0 && kv > 0;
+
+  const int rows = live ? ql * p.G : 0;
+  const bool one_page = p.S % KV_CHUNK == 0;  // a chunk lies in one page
+#pragma unroll 1
+  for (int rb = 0; rb * ROW_BLOCK < rows; ++rb) {
+    const int nch = rb_units(kv, ql, p.G, rb, p.skip_masked, p.sliding_window);
+    const int first = rb_first_chunk(kv, ql, p.G, rb, p.skip_masked, p.sliding_window);
+    if (nch == 0) continue;
+    const int last = first + nch;
+    // the wave's chunks of this block: those of its residue class from `first` on
+    const int row = rb * ROW_BLOCK + n, rrow = row < rows ? row : 0;
+    const int tok = rrow / p.G, g = rrow - tok * p.G;
+    const int pos = kv - ql + (row < rows ? tok : 0);
+    const size_t qrow = (size_t)(q0 + tok) * p.Hq + (size_t)h * p.G + g;
+    bf16x8 q[KS];
+    uint2 rst = {0u, 0u};
+#pragma unroll
+    for (int s = 0; s < KS; ++s) {
+      const int d = 32 * s + 8 * j;
+      const u32x4 w = *(const u32x4*)(p.q + qrow * D + (d < D ? d : 0));
+      q[s] = __builtin_bit_cast(bf16x8, d < D ? w : u32x4{0u, 0u, 0u, 0u});
+    }
+    if constexpr (kFused)
+      if (p.rel_states) rst = *(const uint2*)(p.rel_states + qrow * kRelRows + 4 * j);
+    f32x4 acc[DB];
+#pragma unroll
+    for (int d = 0; d < DB; ++d) acc[d] = f32x4{0.f, 0.f, 0.f, 0.f};
+    float m = -INFINITY, l = 0.f;
+
+    const uint8_t* kbase = a.kb + (size_t)h * a.head;
+    const uint8_t* vbase = a.vb + (size_t)h * a.head;
+    // chunks that every row sees in full, without a soft cap or a window, skip the masks
+    const int pos0 = kv - ql + rb * ROW_BLOCK / p.G;
+    const int plain = p.soft_cap > 0.f || p.sliding_window > 0 ? 0 : ((pos0 + 1 < kv ? pos0 + 1 : kv) / KV_CHUNK);
+    using Half = DirectHalf<MODE, DW>;
+    const int piece = 16 * (lane % Half::kLanes);  // (pieces wholly past D read the row's first piece)
+    const uint8_t* kpiece = kbase + (piece < D * kElem ? piece : 0);
+    const uint8_t* vpiece = vbase + (piece < D * kElem ? piece : 0);
+    auto load = [&](int c, int id, DirectChunk<MODE, DW>& x) {
+      // lane L < 32: the pool row of key L; keys past kv read key kv - 1, whose page id is with its lane
+      const int at = kv - 1 - c * KV_CHUNK < KV_CHUNK - 1 ? kv - 1 - c * KV_CHUNK : KV_CHUNK - 1;
+      const int id_last = rl(id, at);
+      int kt = c * KV_CHUNK + (lane & 31);
+      const bool in_seq = kt < kv;
+      kt = in_seq ? kt : kv - 1;
+      int pg = in_seq ? id : id_last;
+      const bool ok = pg >= 0 && pg < p.P;
+      if (in_seq && !ok) err |= ERR_PAGE;
+      pg = ok ? pg : 0;
+      const int row = (int)((uint32_t)pg * (uint32_t)p.S + (uint32_t)(kt - page(kt) * p.S));
+#pragma unroll
+      for (int l = 0; l < Half::kLoads; ++l) {
+        const int key = Half::kKeys * l + lane / Half::kLanes;
+        const uint64_t off = (uint64_t)(uint32_t)__builtin_amdgcn_ds_bpermute(4 * key, row) * (uint32_t)a.row;
+        const uint8_t *kp = kpiece + off, *vp = vpiece + off;
+        if constexpr (kFused) {
+          if (key >= at && c * KV_CHUNK + at == kv - 1) {  // the step's new token is not in the cache yet
+            const size_t nr = ((size_t)i * p.Hkv + h) * D * 2 + (piece < 2 * D ? piece : 0);
+            kp = (const uint8_t*)p.new_k + nr;
+            vp = (const uint8_t*)p.new_v + nr;
+          }
+        }
+        x.k.w[l] = *(const u32x4*)kp;
+        x.v.w[l] = *(const u32x4*)vp;
+      }
+      if constexpr (MODE == KV_FP8) {
+        x.scale = f32x2{1.f, 1.f};
+        if (p.kv_scales) x.scale = *(const f32x2*)(p.kv_scales + ((size_t)pg * p.Hkv + h) * 2);
+      }
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        if constexpr (MODE == KV_BF16_BIAS) {
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kb = c * KV_CHUNK + 16 * blk + 4 * j + r;
+            x.b[blk][r] = a.bias[(size_t)(h * p.G + g) * a.bias_len + (kb < kv && kb < a.bias_len ? kb : 0)];
+          }
+        }
+        if constexpr (kFused) {
+          const int dist = kv - 1 - (c * KV_CHUNK + 16 * blk + n);
+          const bool in = dist >= 0 && dist < p.rel_extent && p.rel_states;
+#pragma unroll
+          for (int t = 0; t < 4; ++t) x.b[blk][t] = in ? p.rel_proj[(size_t)(4 * j + t) * p.rel_extent + dist] : (uint16_t)0;
+        }
+      }
+    };
+
+    bool fresh = true;  // acc is still zero
+    auto compute = [&](int c, const DirectChunk<MODE, DW>& x) {
+      f32x4 bias[2] = {f32x4{0.f, 0.f, 0.f, 0.f}, f32x4{0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        if constexpr (MODE == KV_BF16_BIAS)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) bias[blk][r] = __builtin_bit_cast(float, (uint32_t)x.b[blk][r] << 16);
+        if constexpr (kFused) {  // P S: P[key][r] = rel_proj[r][distance of key] (0 outside the window), S = rel_states
+          const short4_t af = {(short)x.b[blk][0], (short)x.b[blk][1], (short)x.b[blk][2], (short)x.b[blk][3]};
+          bias[blk] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(af, __builtin_bit_cast(short4_t, rst), bias[blk], 0, 0, 0);
+        }
+      }
+      float ks = p.k_scale, vs = p.v_scale;
+      if constexpr (MODE == KV_FP8) {
+        ks *= x.scale[0];
+        vs *= x.scale[1];
+      }
+      // K to LDS as key rows, S = K Q^T, then V in its place
+      wave_lds_fence();
+      direct_store<MODE, DW, kRowV>(vt, x.k, lane, ks, one_page);
+      wave_lds_fence();
+      f32x4 sc[2];
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk) {
+        sc[blk] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s = 0; s < KS; ++s) sc[blk] = mfma(*(const bf16x8*)(vt + (16 * blk + n) * kRowV + 64 * s + 16 * j), q[s], sc[blk]);
+        if (MODE == KV_FP8 && one_page)  // one K scale (exact codes), on the fp32 scores
+          sc[blk] *= __builtin_bit_cast(float, uni(__builtin_bit_cast(int, ks)));
+      }
+      wave_lds_fence();
+      direct_store<MODE, DW, kRowV>(vt, x.v, lane, vs, false);
+      float y[2][4];
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          y[blk][r] = sc[blk][r] * p.scale_log2;
+          if constexpr (has_bias<MODE>()) y[blk][r] += bias[blk][r] * kLog2e;
+        }
+      if (c >= plain) {
+        if (p.soft_cap > 0.f) {  // soft_cap * tanh(t / soft_cap): sign(t) (1 - z) / (1 + z), z = exp(-2 |t| / soft_cap)
+          const float ec = 2.f * kLog2e / p.soft_cap;
+#pragma unroll
+          for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+              const float t = sc[blk][r] * p.sm_scale, z = __builtin_amdgcn_exp2f(-fabsf(t) * ec);
+              y[blk][r] = copysignf(p.soft_cap * kLog2e * ((1.f - z) / (1.f + z)), t);
+              if constexpr (has_bias<MODE>()) y[blk][r] += bias[blk][r] * kLog2e;
+            }
+        }
+        const int kt0 = c * KV_CHUNK + 4 * j, low = p.sliding_window > 0 ? pos - p.sliding_window : -1;
+#pragma unroll
+        for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            const int kt = kt0 + 16 * blk + r;
+            if (kt > pos || kt <= low) y[blk][r] += p.mask_log2;
+            if (kt >= kv) y[blk][r] = -INFINITY;
+          }
+      }
+      const float mc = rows4_max(fmaxf(fmaxf(fmaxf(y[0][0], y[0][1]), fmaxf(y[0][2], y[0][3])),
+                                       fmaxf(fmaxf(y[1][0], y[1][1]), fmaxf(y[1][2], y[1][3]))));
+      const bool grow = mc > m + kRescaleLog2;  // (lazily moved reference: see unit_softmax)
+      if (__ballot(grow)) {
+        const float mn = grow ? mc : m;
+        const float alpha = __builtin_amdgcn_exp2f(m - (mn == -INFINITY ? 0.f : mn));
+        m = mn;
+        l *= alpha;
+        if (!fresh) {
+#pragma unroll
+          for (int d = 0; d < DB; ++d) acc[d] *= alpha;
+        }
+      }
+      fresh = false;
+      const float mu = m == -INFINITY ? 0.f : m;
+      float e[2][4];
+#pragma unroll
+      for (int blk = 0; blk < 2; ++blk)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) e[blk][r] = __builtin_amdgcn_exp2f(y[blk][r] - mu);
+      l += ((e[0][0] + e[0][1]) + (e[0][2] + e[0][3])) + ((e[1][0] + e[1][1]) + (e[1][2] + e[1][3]));
+      u32x4 pw;
+      pw[0] = pack_bf16x2(e[0][0], e[0][1]);
+      pw[1] = pack_bf16x2(e[0][2], e[0][3]);
+      pw[2] = pack_bf16x2(e[1][0], e[1][1]);
+      pw[3] = pack_bf16x2(e[1][2], e[1][3]);
+      wave_lds_fence();
+      typedef __attribute__((address_space(3))) short4_t* lds_s4;
+      const uint8_t* vb = vt + (4 * j + (n >> 2)) * kRowV + 8 * (n & 3);  // (read_vt_fragments)
+#pragma unroll
+      for (int d = 0; d < DB; ++d) {
+        const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(vb + 32 * d));
+        const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(vb + 16 * kRowV + 32 * d));
+        acc[d] = mfma(__builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7)),
+                      __builtin_bit_cast(bf16x8, pw), acc[d]);
+      }
+    };
+
+    // the wave's chunks, one ahead in flight
+    int c = first + ((wv - first) & (kDirectWaves - 1));
+    const bool used = c < last;
+    if (used) {
+      if (rb > 0 || c != wv) {
+        id0 = load_ids(c);
+        id1 = load_ids(c + kDirectWaves);
+      }
+      DirectChunk<MODE, DW> ca;
+      load(c, id0, ca);
+      if constexpr (kPrefetch) {
+        DirectChunk<MODE, DW> cb;
+        auto turn = [&](const DirectChunk<MODE, DW>& cur, DirectChunk<MODE, DW>& nxt) {
+          const int cn = c + kDirectWaves;
+          const bool more = cn < last;
+          if (more) {
+            load(cn, id1, nxt);
+            id1 = load_ids(cn + kDirectWaves);
+          }
+          compute(c, cur);
+          c = cn;
+          return more;
+        };
+#pragma unroll 1
+        while (turn(ca, cb) && turn(cb, ca)) {
+        }
+      } else {
+#pragma unroll 1
+        for (;;) {
+          compute(c, ca);
+          c += kDirectWaves;
+          if (c >= last) break;
+          load(c, id1, ca);
+          id1 = load_ids(c + kDirectWaves);
+        }
+      }
+    }
+
+    // merge: every wave's (m, l), then its accumulators against the block's reference, row-major in LDS
+    const float lt = rows4_sum(l);
+    const int nrows = rows - rb * ROW_BLOCK < ROW_BLOCK ? rows - rb * ROW_BLOCK : ROW_BLOCK;
+    if (j == 0) *(f32x2*)(sml + (wv * 16 + n) * 2) = f32x2{m, lt};
+    __syncthreads();
+    float M = -INFINITY;
+#pragma unroll
+    for (int w = 0; w < kDirectWaves; ++w) M = fmaxf(M, sml[(w * 16 + n) * 2]);
+    if (used && n < nrows) {
+      const float f = __builtin_amdgcn_exp2f(m - (M == -INFINITY ? 0.f : M));
+      float* o = (float*)vt + n * kRowO + 4 * j;
+#pragma unroll
+      for (int d = 0; d < DB; ++d) *(f32x4*)(o + 16 * d) = acc[d] * f;
+    }
+    __syncthreads();
+    for (int t = threadIdx.x; t < nrows * (DW / 4); t += 64 * kDirectWaves) {
+      const int r = t / (DW / 4), d = 4 * (t - r * (DW / 4));
+      float Mr = -INFINITY, L = 0.f;
+#pragma unroll
+      for (int w = 0; w < kDirectWaves; ++w) Mr = fmaxf(Mr, sml[(w * 16 + r) * 2]);
+      const float mu = Mr == -INFINITY ? 0.f : Mr;
+      f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int w = 0; w < kDirectWaves; ++w) {
+        // wave w has chunks of this block iff its residue class meets [first, last)
+        const int miss = (w - first) & (kDirectWaves - 1);
+        if (first + miss < last) {
+          o += *(const f32x4*)((const float*)(smem + w * kRegion) + r * kRowO + d);
+          L += sml[(w * 16 + r) * 2 + 1] * __builtin_amdgcn_exp2f(sml[(w * 16 + r) * 2] - mu);
+        }
+      }
+      const float inv = 1.f / L;
+      const int orow = rb * ROW_BLOCK + r, ot = orow / p.G, og = orow - ot * p.G;
+      u32x2 w2;
+      w2[0] = pack_bf16x2(o[0] * inv, o[1] * inv);
+      w2[1] = pack_bf16x2(o[2] * inv, o[3] * inv);
+      if (d < D) *(u32x2*)(p.out + ((size_t)(q0 + ot) * p.Hq + (size_t)h * p.G + og) * D + d) = w2;
+    }
+    __syncthreads();  // the regions are free for the next row block
+  }
+
+  if constexpr (kFused) {  // the new token's rows of this kv head (fused_store_token)
+    if (live && store && wv == 0 && lane < 32) {
+      const int kt = kv - 1, which = lane >> 4, d = 8 * (lane & 15);
+      const int pg = p.page_indices[prow + page(kt)];
+      if (pg >= 0 && pg < p.P) {
+        const uint16_t* src = (which ? p.new_v : p.new_k) + ((size_t)i * p.Hkv + h) * D;
+        const u32x4 w = *(const u32x4*)(src + (d < D ? d : 0));
+        uint8_t* dst = (uint8_t*)(which ? a.vb : a.kb) + ((long long)pg * p.S + (kt - page(kt) * p.S)) * a.row + (long long)h * a.head;
+        *(u32x4*)(dst + 2 * d) = d < D ? w : u32x4{0u, 0u, 0u, 0u};
+      } else {
+        err |= ERR_PAGE;
+      }
+    }
+  } else if constexpr (!kV1) {  // rows at or past cu_q_lens[num_seqs] belong to no sequence: zero them
+    int tv = uni(p.cu_q_lens[nseq]);
+    tv = tv < 0 ? 0 : (tv > p.T ? p.T : tv);
+    const size_t f = (size_t)tv * p.Hq * D / 8, e = (size_t)p.T * p.Hq * D / 8;
+    for (size_t k = f + (size_t)blockIdx.x * blockDim.x + threadIdx.x; k < e; k += (size_t)gridDim.x * blockDim.x)
+      ((u32x4*)p.out)[k] = u32x4{0u, 0u, 0u, 0u};
+  }
+  if (err) atomicOr(p.err, err);
+}
+
+// Whether a call runs as one workgroup per (sequence, kv head) in a single launch (bounds: see the
+// kernel), with no schedule knob asked for.
+bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
+  const long long cap = (long long)s->pages_per_seq * s->page_size;
+  return s->num_tokens <= s->max_num_seqs && cap <= kDirectMaxKeys &&
+         cap * (s->head_dim < 64 ? 64 : s->head_dim) <= kDirectElems &&
+         (long long)s->max_num_seqs * s->num_kv_heads <= kDirectGroups &&
+         (o->waves_per_cu == 0 || o->waves_per_cu == kMaxWavesPerCU) &&
+         (unsigned long long)s->total_pages * s->page_size <= 0xffffffffull;  // pool rows in 32 bits
+}
+
+template <int MODE, int DW>
+void launch_direct_kernel(const Params& p, DirectArgs a, hipStream_t st) {
+  a.pmagic = (uint32_t)(((1ull << 31) + p.S - 1) / p.S);
+  constexpr size_t lds = kDirectWaves * (KV_CHUNK * (2 * DW + 32) + 16 * 2 * sizeof(float));
+  hipLaunchKernelGGL((rpa_attn_kernel_direct<MODE, DW>), dim3(p.Nmax * p.Hkv), dim3(64 * kDirectWaves), lds, st, p, a);
+}
+
+template <int MODE>
+void launch_direct_mode(const Params& p, const DirectArgs& a, hipStream_t st) {
+  if (p.D <= 64) launch_direct_kernel<MODE, 64>(p, a, st);
+  else if (p.D <= 128) launch_direct_kernel<MODE, 128>(p, a, st);
+  else if constexpr (!has_bias<MODE>()) launch_direct_kernel<MODE, 256>(p, a, st);
+}
+
+// ---------------------------------------------------------------------------------------------
 // gather probe
 // ---------------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void rpa_gather_kernel(Params p, uint8_t* dense, long long dense_rows, int elem) {
@@ -4928,6 +5390,27 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     if (kv_scales) return fail(RPA_E_INVALID, "kv_scales is only used with fp8 kv_pages");
     if (opt->has_k_scale || opt->has_v_scale) mode = KV_BF16_SCALED;
   }
+  hipStream_t st = (hipStream_t)stream;
+  if (direct_call(shape, opt) && mode != KV_BF16_BIAS) {
+    const int elem = mode == KV_FP8 ? 1 : 2, width = fz ? kD : p.D;  // (the fused step's cache rows are kD wide)
+    DirectArgs a;
+    memset(&a, 0, sizeof(a));
+    a.kb = p.kv;
+    a.vb = p.kv + (size_t)width * elem;
+    a.row = (long long)2 * p.Hkv * width * elem;
+    a.head = 2 * width * elem;
+    if (ev_begin && hipEventRecord((hipEvent_t)ev_begin, st) != hipSuccess)
+      return fail(RPA_E_HIP, "hipEventRecord(begin) failed");
+    if (mode == KV_BF16_FUSED) launch_direct_mode<KV_BF16_FUSED>(p, a, st);
+    else if (mode == KV_FP8) launch_direct_mode<KV_FP8>(p, a, st);
+    else if (mode == KV_BF16_SCALED) launch_direct_mode<KV_BF16_SCALED>(p, a, st);
+    else launch_direct_mode<KV_BF16>(p, a, st);
+    const hipError_t de = hipGetLastError();
+    if (de != hipSuccess) return fail(RPA_E_HIP, std::string("attention launch failed: ") + hipGetErrorString(de));
+    if (ev_end && hipEventRecord((hipEvent_t)ev_end, st) != hipSuccess)
+      return fail(RPA_E_HIP, "hipEventRecord(end) failed");
+    return RPA_OK;
+  }
   resolve_layout(p, mode, shape, opt, (uintptr_t)kv_pages % 16 == 0);
   const int waves = p.co ? kCoWaves : p.HG;  // per workgroup
   p.grid = grid_for_call(d, mode, waves, opt->waves_per_cu);
@@ -4940,7 +5423,6 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     p.co_split_max = d.cus;
     p.co_desc = (CoDesc*)((uint8_t*)workspace + w.co_desc);
   }
-  hipStream_t st = (hipStream_t)stream;
   if (ev_begin && hipEventRecord((hipEvent_t)ev_begin, st) != hipSuccess)
     return fail(RPA_E_HIP, "hipEventRecord(begin) failed");
   const bool upg = p.S % KV_CHUNK == 0;
@@ -5035,6 +5517,11 @@ int rpa_attention_grid(const rpa_shape_t* shape, const rpa_options_t* opt, int32
   if (rc) return rc;
   if (cus < 0) return fail(RPA_E_INVALID, "cus must be >= 0");
   Params p = base_params(shape);
+  if (direct_call(shape, opt)) {
+    *grid = p.Nmax * p.Hkv;
+    *waves_per_workgroup = kDirectWaves;
+    return RPA_OK;
+  }
   const float mask = opt->has_mask_value ? opt->mask_value : kDefaultMask;
   p.skip_masked = mask <= -1e30f;
   int mode = KV_BF16;
@@ -5170,6 +5657,36 @@ int rpa_inkling_decode(const rpa_inkling_shape_t* f, float sm_scale, const void*
   a.L = f->bias_len;
   a.vec = ((uintptr_t)key_cache | (uintptr_t)value_cache) % 16 == 0 && a.D % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
+  if (a.vec && (long long)f->pages_per_seq * f->page_size <= kDirectMaxKeys &&
+      (unsigned long long)f->total_pages * f->page_size <= 0xffffffffull) {
+    // one launch over the caller's own caches (nothing packed, padded or merged)
+    const rpa_shape_t ds = v1_rpa_shape(f);
+    Params p = base_params(&ds);
+    p.D = f->head_dim;
+    p.q = a.q;
+    p.kv = (const uint8_t*)a.kc;
+    p.kv_lens = sequence_lengths;
+    p.page_indices = page_table;
+    p.fused_nseq = a.B;
+    p.out = (uint16_t*)out;
+    p.err = (int32_t*)workspace;
+    p.sm_scale = sm_scale;
+    p.scale_log2 = sm_scale * kLog2e;
+    p.mask_log2 = kDefaultMask * kLog2e;
+    p.skip_masked = true;
+    p.k_scale = p.v_scale = 1.f;
+    DirectArgs d1;
+    d1.kb = (const uint8_t*)a.kc;
+    d1.vb = (const uint8_t*)a.vc;
+    d1.row = (long long)a.Hkv * a.D * 2;
+    d1.head = a.D * 2;
+    d1.bias = a.bias;
+    d1.bias_len = a.L;
+    launch_direct_mode<KV_BF16_BIAS>(p, d1, st);
+    const hipError_t de = hipGetLastError();
+    if (de != hipSuccess) return fail(RPA_E_HIP, std::string("inkling launch failed: ") + hipGetErrorString(de));
+    return RPA_OK;
+  }
   const long long work = (long long)a.P * a.S * 2 * a.Hkv * (kD / 8);
   long long blocks = (work + 255) / 256;
   blocks = blocks < 1 ? 1 : (blocks > 4096 ? 4096 : blocks);
