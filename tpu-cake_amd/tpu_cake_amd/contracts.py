@@ -341,6 +341,22 @@ def _work_split(kv_lens, q_lens, hq: int, hkv: int, kv_dtype: str, prefill_tiles
                 prefill_chunk_steps=round(steps))
 
 
+DIRECT_ELEMS, DIRECT_GROUPS, DIRECT_MAX_KEYS, DIRECT_WAVES = 1024 * 128, 512, 4096, 8  # csrc/rpa_kernels.hip, direct_call
+
+
+def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, table_keys: int) -> bool:
+    """Whether a call runs in one launch, a workgroup per (sequence, kv head) (direct_call with the
+    default knobs); table_keys: the keys a sequence's page table holds."""
+    return (num_tokens <= max_num_seqs and table_keys <= DIRECT_MAX_KEYS
+            and table_keys * max(head_dim, 64) <= DIRECT_ELEMS and max_num_seqs * hkv <= DIRECT_GROUPS)
+
+
+def _direct_line(seqs: int, hkv: int, what: str) -> str:
+    return (f"launch (short page tables) = rpa_attn_kernel_direct: grid {seqs * hkv} x block {64 * DIRECT_WAVES} (one "
+            f"workgroup per (sequence, kv head), its waves' states merged in LDS; {what}); longer page tables or more "
+            "pairs take the launches below")
+
+
 def _plan_text(name: str, lines: list[str]) -> str:
     return "\n".join([f"mi355x-rpa launch plan v1: {name}"] + lines) + "\n"
 
@@ -395,6 +411,8 @@ def _operator_workload(cfg: str) -> tuple[str, WorkloadContract, dict]:
         f"sequences = {m.num_seqs}; query tokens = {m.num_tokens}; sum kv_len = {int(sum(m.kv_lens))}",
         f"heads = Hq {m.num_q_heads} / Hkv {m.num_kv_heads} (G {split['group']}); head_dim {m.head_dim}; "
         f"page_size {m.page_size}; pool pages {m.pool_pages}; pages per sequence {m.pages_per_seq}",
+        *([_direct_line(m.num_seqs, m.num_kv_heads, "this call's form")]
+          if direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size) else []),
         f"launch 0 = rpa_attn_kernel<{mode}, page ids per {'chunk' if upg else 'key'}"
         f"{', co-resident' if co else ''}>: "
         f"grid {split['grid']} x block {64 * hg} ({hg} kv heads per workgroup, one wave each; "
@@ -452,9 +470,10 @@ def _inkling_v1_workload() -> tuple[str, WorkloadContract, dict]:
     lines = [
         "description = v1 Inkling decode contract: separate K/V caches, additive relative bias [H, L] by key "
         "position, scale 1/D (workloads/inkling_rpa.py:37-73, :693-722)",
-        "entry = rpa_inkling_decode (include/rpa.h); one call = the four launches below, stream-ordered",
+        "entry = rpa_inkling_decode (include/rpa.h); one call = one launch, or the four below, stream-ordered",
         f"sequences = {B} (one query token each); heads = Hq {H} / Hkv {H}; head_dim {D} (rows padded to 128); "
         f"page_size {S}; pool pages {P}; pages per sequence {MP}",
+        _direct_line(B, H, "over the caller's own caches, the bias by key position: this call's form"),
         "launch 0 = rpa_inkling_v1_prep_kernel: grid-stride; packs the K/V caches into the combined "
         "[P, S, 2H, 128] layout, writes the bias table by key position, cu_q = 0..B, num_seqs, padded queries",
         f"launch 1 = rpa_attn_kernel<KV_BF16_BIAS>: grid {split['grid']} x block {64 * split['heads_per_workgroup']}; "
@@ -500,9 +519,10 @@ def _inkling_fused_workload() -> tuple[str, WorkloadContract, dict]:
         "relative-position bias relative_states . relative_projection for distances < E, scale 1/D "
         "(workloads/inkling_rpa.py:471-589)",
         "entry = rpa_inkling_fused_decode (include/rpa.h), after the host preflight "
-        "(rpa_lowering.py:71-128); one call = the two launches below, stream-ordered",
+        "(rpa_lowering.py:71-128); one call = one launch, or the two below, stream-ordered",
         f"tokens = sequences = {N}; heads = Hq {Hq} / Hkv {Hkv}; head_dim {D} (cache rows padded to 128); "
         f"page_size {S}; pages {P}; relative states R {R}, extent E {E}",
+        _direct_line(N, Hkv, "which stores the new K/V rows too: this call's form"),
         f"launch 0 = rpa_attn_kernel<KV_BF16_FUSED, page ids per key>: grid {split['grid']} x block "
         f"{64 * split['heads_per_workgroup']}; sequence i's pages from page_indices[cu_kv_lens[i] / S], its new "
         "token's K/V read from keys/values, queries and output rows D wide, the relative bias formed in the "
