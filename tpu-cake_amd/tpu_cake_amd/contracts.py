@@ -519,7 +519,7 @@ def _inkling_fused_workload() -> tuple[str, WorkloadContract, dict]:
         "relative-position bias relative_states . relative_projection for distances < E, scale 1/D "
         "(workloads/inkling_rpa.py:471-589)",
         "entry = rpa_inkling_fused_decode (include/rpa.h), after the host preflight "
-        "(rpa_lowering.py:71-128); one call = one launch, or the two below, stream-ordered",
+        "(rpa_lowering.py:71-128); one call = the two launches below, stream-ordered, or one launch",
         f"tokens = sequences = {N}; heads = Hq {Hq} / Hkv {Hkv}; head_dim {D} (cache rows padded to 128); "
         f"page_size {S}; pages {P}; relative states R {R}, extent E {E}",
         _direct_line(N, Hkv, "which stores the new K/V rows too: this call's form"),
