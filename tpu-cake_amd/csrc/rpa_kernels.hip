@@ -652,7 +652,8 @@ __device__ __forceinline__ size_t page_row(const Params& p, const Cursor& x) {
   return (size_t)x.i * p.PPS;
 }
 
-template <int MODE, bool UPG>
+// LINE: the full-line path (LinePath).
+template <int MODE, bool UPG, bool LINE>
 __device__ __forceinline__ Pages load_pages(const Params& p, const Cursor& x, int n) {
   Pages r;
   if constexpr (UPG) {
@@ -665,7 +666,7 @@ __device__ __forceinline__ Pages load_pages(const Params& p, const Cursor& x, in
   const bool live = x.nch > 0;
   const int last = x.kv_len > 0 ? x.kv_len - 1 : 0;
   const size_t row = live ? page_row<MODE>(p, x) : 0;
-  if constexpr (MODE == KV_BF16_FUSED) {
+  if constexpr (LINE) {
     // the full-line path with pages smaller than a unit: lane L's key key0 + L % 32 -- its page id
     // and its slot in the page (line_addr)
     int kt = x.key0() + (n + 16 * ((threadIdx.x >> 4) & 1));
@@ -1193,7 +1194,7 @@ __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n,
     advance<MODE>(p, nseq, lane, win, ahead, err);
   else
     ahead.nch = 0;
-  const Pages pg_ahead = load_pages<MODE, UPG>(p, ahead, n);
+  const Pages pg_ahead = load_pages<MODE, UPG, false>(p, ahead, n);
   const UnitAddr nx_addr = unit_addr(p, nxt, pg_nxt, n, j, wv, err, D);
   // keep the workgroup's waves (the kv heads of one group) in step, so the heads' slices of the
   // same keys reach the memory system together (a workgroup of several workers has nothing to keep)
@@ -1216,7 +1217,7 @@ __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n,
 
 
 // ---------------------------------------------------------------------------------------------
-// full-line decode path (bf16 KV, page size a multiple of 32)
+// full-line decode path (bf16 KV)
 // ---------------------------------------------------------------------------------------------
 // The path above loads K and V straight into the MFMA operand layout: 16 keys x 64 bytes per load
 // instruction, half of every 128-byte line.  Here a wave loads its kv head's K (then V) rows of a
@@ -1229,10 +1230,15 @@ __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n,
 // K of the next unit lands while this unit's K is read from the tile, V of the next unit is loaded
 // once this unit's V is stored.
 
+// Page sizes that are not a multiple of 32 (not UPG) take it too, each lane finding its key's pool
+// row in the lane that looked the key's page up (line_addr).  Pages of 16, against the operand
+// layout above, 64 sequences of ~2048 keys, 8 kv heads: 128-dim heads 121 -> 107 us, 64-dim 106 ->
+// 59 (rows of 64 elements fixed at compile time), 256-dim (4 kv heads) 132 -> 108, a window of 512
+// 42 -> 37.  fp8 has its own layout, and the v1 bias there is added in the operand layout.
 template <int MODE, bool UPG>
 struct LinePath {
-  static constexpr bool on =
-      MODE == KV_BF16_FUSED || (UPG && (MODE == KV_BF16 || MODE == KV_BF16_SCALED || MODE == KV_BF16_BIAS));
+  static constexpr bool on = MODE == KV_BF16 || MODE == KV_BF16_SCALED || MODE == KV_BF16_FUSED ||
+                             (MODE == KV_BF16_BIAS && UPG);
 };
 
 struct LineRegs {
@@ -1259,7 +1265,7 @@ struct LineAddr {
   int bias_at;  // as UnitAddr
   int knew;       // fused step: the unit's key (0..31) read from new_k / new_v instead, -1 = none
   size_t newoff;  // fused step: element index of this lane's dims of that key's row in new_k / new_v
-  int row;        // fused step, pages smaller than a unit: pool row (page * S + slot) of key lane % 32
+  uint32_t row;   // pages smaller than a unit: pool row (page * S + slot) of key lane % 32
 };
 
 template <int MODE, bool UPG = true, int DN = 0>
@@ -1268,22 +1274,23 @@ __device__ __forceinline__ LineAddr line_addr(const Params& p, const Cursor& x, 
   LineAddr a;
   const bool live = x.nch > 0;
   if constexpr (!UPG) {
-    // (the fused step only: D = kD, head v = h * HG + wv) pages smaller than a unit: the keys of
-    // one load instruction may lie in different pages; lane L checks the page of key L % 32 and
-    // keeps its pool row, which load_lines hands to the lanes that read that key
-    static_assert(MODE == KV_BF16_FUSED, "per-key pages on the full-line path: the fused step only");
+    // pages smaller than a unit: the keys of one load instruction may lie in different pages; lane L
+    // checks the page of key L % 32 and keeps its pool row, which load_lines hands to the lanes that
+    // read that key
     const int v = live ? x.h * p.HG + wv : 0;
     const bool in_seq = live && x.key0() + (lane & 31) < x.kv_len;
     const bool pg_ok = pages.pg[0] >= 0 && pages.pg[0] < p.P;
     if (in_seq && !pg_ok) err |= ERR_PAGE;
-    a.row = (pg_ok ? pages.pg[0] : 0) * p.S + pages.pg[1];
-    a.e0 = (size_t)(2 * v) * kD + 8 * (lane & 15);
+    // (a row holds at least 2 x 32 elements: 2^32 of them would be a pool of 512 GiB)
+    a.row = (uint32_t)(pg_ok ? pages.pg[0] : 0) * (uint32_t)p.S + (uint32_t)pages.pg[1];
+    const int piece = 8 * (lane & (Lines<DN>::lanes - 1));  // (pieces past a narrow row: its first one)
+    a.e0 = (size_t)(2 * real_head(v, D)) * D + half_offset(v, D) + (D == kD || piece < D ? piece : 0);
     const int k = live ? x.kv_len - 1 - x.key0() : 0;
     a.kmax = k < KV_CHUNK - 1 ? k : KV_CHUNK - 1;
     a.bias_at = 0;
     a.knew = -1;
     a.newoff = 0;
-    if (live && k < KV_CHUNK) {
+    if (MODE == KV_BF16_FUSED && live && k < KV_CHUNK) {
       a.knew = k;
       a.newoff = ((size_t)x.i * p.Hkv + v) * p.D + (8 * (lane & 15) < p.D ? 8 * (lane & 15) : 0);
     }
@@ -1316,28 +1323,20 @@ __device__ __forceinline__ void load_lines(const Params& p, const LineAddr& a, i
                                            int D = kD) {
   const uint16_t* kv = (const uint16_t*)p.kv + a.e0 + (size_t)which * D;
   const size_t row = (size_t)(2 * p.Hkv) * D;
-  if constexpr (DN != 0) {
-    static_assert(UPG && MODE != KV_BF16_FUSED, "narrow rows: whole-page units, cache rows of D");
-    using L = Lines<DN>;
-#pragma unroll
-    for (int i = 0; i < L::loads; ++i) {
-      int key = L::keys * i + lane / L::lanes;
-      key = key < a.kmax ? key : a.kmax;
-      r.w[i] = ld_stream((const u32x4*)(kv + (size_t)key * row));
-    }
-    return;
-  }
+  static_assert(DN == 0 || MODE != KV_BF16_FUSED, "narrow rows: cache rows of D");
   const uint16_t* nw = nullptr;
   if constexpr (MODE == KV_BF16_FUSED) nw = (which ? p.new_v : p.new_k) + a.newoff;
+  using L = Lines<DN>;
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    int key = 4 * i + (lane >> 4);
+  for (int i = 0; i < L::loads; ++i) {
+    int key = L::keys * i + lane / L::lanes;
     key = key < a.kmax ? key : a.kmax;
     const uint16_t* src;
-    if constexpr (UPG)
+    if constexpr (UPG) {
       src = kv + (size_t)key * row;
-    else  // the key's pool row, from lane key (line_addr)
-      src = kv + (size_t)__builtin_amdgcn_ds_bpermute(4 * key, a.row) * row;
+    } else {  // the key's pool row, from lane key (line_addr)
+      src = kv + (size_t)(uint32_t)__builtin_amdgcn_ds_bpermute(4 * key, (int)a.row) * row;
+    }
     if constexpr (MODE == KV_BF16_FUSED) src = key == a.knew ? nw : src;  // the step's new token
     r.w[i] = ld_stream((const u32x4*)src);
   }
@@ -1490,7 +1489,7 @@ __device__ __forceinline__ void step_line(const Params& p, int nseq, int lane, i
     advance<MODE>(p, nseq, lane, win, ahead, err);
   else
     ahead.nch = 0;
-  const Pages pg_ahead = load_pages<MODE, UPG>(p, ahead, n);
+  const Pages pg_ahead = load_pages<MODE, UPG, true>(p, ahead, n);
   const LineAddr nx_addr = line_addr<MODE, UPG, DN>(p, nxt, pg_nxt, lane, n, j, wv, err, D);
   if (!CO || p.lockstep) __syncthreads();
   load_lines<MODE, UPG, DN>(p, nx_addr, lane, 0, k, D);  // the next unit's K (this unit's K is in the tile)
@@ -2998,7 +2997,7 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
 // (Lines<DN>).
 template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rpa_attn_kernel(Params p) {
-  static_assert(DN == 0 || (NW && UPG && (DN == 32 || DN == 64)), "DN: a narrow instantiation of 32 or 64");
+  static_assert(DN == 0 || (NW && (DN == 64 || (UPG && DN == 32))), "DN: a narrow instantiation of 32 or 64");
   static_assert(!CO || co_tiles<MODE>(), "CO: a mode with co-resident tiles");
   static_assert(!(CO && NW) || DT == 64, "a narrow co-resident instantiation: 64-dim heads");
   constexpr bool kTiles = CO ? true : NW ? false : MODE == KV_BF16;  // a prefill-tile role exists
@@ -3180,9 +3179,10 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         advance<MODE>(p, nseq, lane, win, nxt, err);
       else
         nxt.nch = 0;
-      const Pages pg_cur = load_pages<MODE, UPG>(p, cur, n);
-      Pages pg_nxt = load_pages<MODE, UPG>(p, nxt, n);
-      if constexpr (LinePath<MODE, UPG>::on) {
+      constexpr bool kLine = LinePath<MODE, UPG>::on;
+      const Pages pg_cur = load_pages<MODE, UPG, kLine>(p, cur, n);
+      Pages pg_nxt = load_pages<MODE, UPG, kLine>(p, nxt, n);
+      if constexpr (kLine) {
         LineRegs k, v;
         f32x4 bias[2];
         LineBias bias_in;
@@ -5445,7 +5445,7 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_FP8, false, true, true, 0, 64>), grid, block, lds, st, p);
     } else {
       if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true, true, 64, 64>), grid, block, lds, st, p);
-      else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true, true, 0, 64>), grid, block, lds, st, p);
+      else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true, true, 64, 64>), grid, block, lds, st, p);
     }
   } else if (p.D != kD) {  // another head dim (decode role only)
     if (mode == KV_FP8) {
@@ -5456,11 +5456,13 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
       if (upg && p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, false, true, 64>), grid, block, lds, st, p);
       else if (upg && p.D == 32) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, false, true, 32>), grid, block, lds, st, p);
       else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, false, true>), grid, block, lds, st, p);
+      else if (p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, true, 64>), grid, block, lds, st, p);
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, true>), grid, block, lds, st, p);
     } else {
       if (upg && p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true, 64>), grid, block, lds, st, p);
       else if (upg && p.D == 32) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true, 32>), grid, block, lds, st, p);
       else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true>), grid, block, lds, st, p);
+      else if (p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true, 64>), grid, block, lds, st, p);
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true>), grid, block, lds, st, p);
     }
   } else if (mode == KV_FP8) {
