@@ -395,3 +395,20 @@ def test_search_summary_markdown(tmp_path):
     res = search.run_search(tmp_path, c, runner=_FakeRunner(case, {0.0: 100, 0.25: 90}), checker=_checker, case=case)
     md = search.summary_markdown(res, "python -m tpu_cake_amd.search ...")
     assert "| pf25 |" in md and "confirmed winner: pf25" in md and "Confirmation (2 paired rounds)" in md
+
+
+def test_small_calls_profile_has_no_combine_launch(tmp_path):
+    """A call that runs in one launch is accepted by the kernels it launches; the others still need both."""
+    assert evidence.call_kernels("c1") == ("rpa_attn_kernel",)
+    for config in ("c2", "c3", "c4", "c5", "c2w", "c2d64"):
+        assert evidence.call_kernels(config) == evidence.KERNELS
+    d = tmp_path / "t"
+    d.mkdir()
+    (d / "run_kernel_stats.csv").write_text(
+        '"Name","Calls","TotalDurationNs","AverageNs","Percentage","MinNs","MaxNs","StdDev"\n'
+        '"void rpa::(anonymous namespace)::rpa_attn_kernel_direct<0, 128>(Params, DirectArgs)",10,10000,1000,99,900,1100,10\n')
+    prof = evidence.inspect_profile(d)
+    assert evidence.assess_profile(prof, dispatches=10, kernels=evidence.call_kernels("c1"))["accepted"]
+    assert not evidence.assess_profile(prof, dispatches=10, kernels=evidence.call_kernels("c2"))["accepted"]
+    from tpu_cake_amd import contracts
+    assert contracts.experiment("mi355x-rpa-c1").profile.required_timed_hlo_markers == ("rpa_attn_kernel_direct",)

@@ -4159,8 +4159,9 @@ __device__ __forceinline__ void direct_store(uint8_t* vt, const DirectHalf<MODE,
 
 // MODE KV_BF16_BIAS: the v1 contract.
 template <int MODE, int DW>
-__global__ __launch_bounds__(64 * kDirectWaves) __attribute__((amdgpu_waves_per_eu(2, 2))) void
-rpa_attn_kernel_direct(Params p, DirectArgs a) {
+__attribute__((amdgpu_waves_per_eu(2, 2))) __launch_bounds__(64 * kDirectWaves)
+__global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
+  RPA_TL(const long long tl_t0 = tl_clock(); tl_begin(); tl_set(TL_START, tl_t0);)
   constexpr int KS = DW / 32, DB = DW / 16;
   constexpr int kRowV = 2 * DW + 32;                 // V region: 32 key rows (conflict-free transposing reads)
   constexpr int kRegion = KV_CHUNK * kRowV;          // ... and, after the chunks, 16 rows of DW + 4 floats
@@ -4516,6 +4517,7 @@ rpa_attn_kernel_direct(Params p, DirectArgs a) {
       ((u32x4*)p.out)[k] = u32x4{0u, 0u, 0u, 0u};
   }
   if (err) atomicOr(p.err, err);
+  RPA_TL(tl_set(TL_END, tl_clock());)
 }
 
 // Whether a call runs as one workgroup per (sequence, kv head) in a single launch (bounds: see the

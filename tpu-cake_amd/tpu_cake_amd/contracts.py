@@ -300,9 +300,10 @@ CO_WAVES = 4  # the co-resident layout's workgroups (csrc/rpa_kernels.hip, kCoWa
 
 def co_resident(head_dim: int, hkv: int, group: int, page_size: int, num_tokens: int, max_num_seqs: int,
                 kv_dtype: str) -> bool:
-    """Whether a call takes the co-resident layout (resolve_layout with the default knobs): 128-dim
-    heads, bf16 or fp8 KV, page size a multiple of 32, Hkv a multiple of 4, and a batch that can hold
-    a sequence of 16 query tokens."""
+    """Whether a call takes the co-resident layout in the form of the planned workloads (resolve_layout
+    with the default knobs; it has others for 64-dim heads and other page sizes and kv head counts):
+    128-dim heads, bf16 or fp8 KV, page size a multiple of 32, Hkv a multiple of 4, and a batch that
+    can hold a sequence of 16 query tokens."""
     return (head_dim == 128 and kv_dtype in ("bf16", "fp8") and page_size % KV_CHUNK == 0
             and hkv % CO_WAVES == 0 and group <= 32 * CO_WAVES and num_tokens >= max_num_seqs + 15)
 
@@ -400,19 +401,19 @@ def _operator_workload(cfg: str) -> tuple[str, WorkloadContract, dict]:
     unit_bytes = hg * KV_CHUNK * 2 * m.head_dim * (1 if m.kv_dtype == "fp8" else 2)
     mode = "KV_FP8" if m.kv_dtype == "fp8" else "KV_BF16"
     upg = m.page_size % KV_CHUNK == 0
-    line = upg and m.kv_dtype != "fp8"
+    line = m.kv_dtype != "fp8"
     floor_hbm = fl["hbm_s"] * 1e6
     floor_mfma = fl["mfma_s"] * 1e6
     half = split["grid"] // 2
     fixed = co and split["prefill_workgroups"] == half and half % 8 == 0
+    direct = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size)
     lines = [
         f"description = {CONFIG_DESCRIPTIONS[cfg]}",
         "entry = rpa_ragged_paged_attention (include/rpa.h); one call = the two launches below, stream-ordered",
         f"sequences = {m.num_seqs}; query tokens = {m.num_tokens}; sum kv_len = {int(sum(m.kv_lens))}",
         f"heads = Hq {m.num_q_heads} / Hkv {m.num_kv_heads} (G {split['group']}); head_dim {m.head_dim}; "
         f"page_size {m.page_size}; pool pages {m.pool_pages}; pages per sequence {m.pages_per_seq}",
-        *([_direct_line(m.num_seqs, m.num_kv_heads, "this call's form")]
-          if direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size) else []),
+        *([_direct_line(m.num_seqs, m.num_kv_heads, "this call's form")] if direct else []),
         f"launch 0 = rpa_attn_kernel<{mode}, page ids per {'chunk' if upg else 'key'}"
         f"{', co-resident' if co else ''}>: "
         f"grid {split['grid']} x block {64 * hg} ({hg} kv heads per workgroup, one wave each; "
@@ -444,7 +445,8 @@ def _operator_workload(cfg: str) -> tuple[str, WorkloadContract, dict]:
         f"QK/PV {work.flops} FLOP (prefill rows {flops})",
         f"roofline floor = HBM {floor_hbm:.2f} us; MFMA {floor_mfma:.2f} us; bound = {fl['bound']}",
     ]
-    return _plan_text(f"mi355x-rpa-{cfg}", lines), contract, dict(kernels=("rpa_attn_kernel", "rpa_combine_kernel"))
+    kernels = ("rpa_attn_kernel_direct",) if direct else ("rpa_attn_kernel", "rpa_combine_kernel")
+    return _plan_text(f"mi355x-rpa-{cfg}", lines), contract, dict(kernels=kernels)
 
 
 def _inkling_v1_workload() -> tuple[str, WorkloadContract, dict]:
@@ -482,7 +484,7 @@ def _inkling_v1_workload() -> tuple[str, WorkloadContract, dict]:
         f"{64 * combine_waves(split['group'])}",
         "launch 3 = rpa_fused_unpad_kernel: output rows 128 -> D",
     ]
-    kernels = ("rpa_inkling_v1_prep_kernel", "rpa_attn_kernel", "rpa_combine_kernel", "rpa_fused_unpad_kernel")
+    kernels = ("rpa_attn_kernel_direct",)
     return _plan_text("mi355x-inkling-rpa", lines), contract, dict(kernels=kernels)
 
 
@@ -531,7 +533,7 @@ def _inkling_fused_workload() -> tuple[str, WorkloadContract, dict]:
         f" x block {64 * combine_waves(split['group'])}; the last N workgroups store each sequence's new K/V rows "
         "in its cache slot",
     ]
-    kernels = ("rpa_attn_kernel", "rpa_combine_kernel")
+    kernels = ("rpa_attn_kernel_direct",)
     return _plan_text("mi355x-inkling-fused-rpa", lines), contract, dict(kernels=kernels)
 
 

@@ -129,12 +129,23 @@ def inspect_profile(path) -> dict:
     return {"kernels": kernels, "counters": counters, "counter_dispatches": dispatches, "files": files}
 
 
-def assess_profile(profile: dict, *, dispatches: int, counters: tuple = ()) -> dict:
+def call_kernels(config: str) -> tuple:
+    """The kernels (by ``_kernel_key``) one call of a configuration launches: small calls have no
+    combine launch."""
+    from .contracts import direct_call
+    from .workloads import make_config_meta_for
+
+    m, _ = make_config_meta_for(config)
+    small = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size)
+    return KERNELS[:1] if small else KERNELS
+
+
+def assess_profile(profile: dict, *, dispatches: int, counters: tuple = (), kernels: tuple = KERNELS) -> dict:
     """Accept a profile if every kernel of the call was captured at least ``dispatches`` times
     (the timed steps) and, for a counters run, every named counter was read for the attention
     kernel (a counters run names the HBM counters and the MFMA-activity ones)."""
     reasons = []
-    for k in KERNELS:
+    for k in kernels:
         calls = profile["kernels"].get(k, {}).get("calls", 0)
         if counters:  # a counters run captures dispatches through its counter rows
             calls = profile.get("counter_dispatches", {}).get(k, 0)
@@ -243,7 +254,8 @@ def run_profiled(root, mode: str, config: str, steps: int, warmup: int) -> dict:
     steps_res = json.loads((phase_root / "steps.json").read_text())
     prof = inspect_profile(phase_root)
     assessment = assess_profile(prof, dispatches=steps,
-                                counters=COUNTERS + MFMA_COUNTERS if mode == "counters" else ())
+                                counters=COUNTERS + MFMA_COUNTERS if mode == "counters" else (),
+                                kernels=call_kernels(config))
     body = {**steps_res, "profile": prof, "assessment": assessment, "passed": assessment["accepted"]}
     return _write_result(phase_root, mode, body)
 
