@@ -2458,16 +2458,12 @@ struct CoTile {
 #pragma unroll
         for (int i = 0; i < 16; ++i) x[i] = s[i] * sl2;
       } else {
-        // soft_cap * tanh(t / soft_cap) with tanh(y) = sign(y) (1 - z) / (1 + z), z = exp(-2 |y|)
         const float sm = L::kFp8 && UPG ? p.sm_scale * uni_f(ksc) : p.sm_scale;
-        const float ec = p.soft_cap > 0.f ? -2.f * kLog2e * sm / p.soft_cap : 0.f;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
           float xv = s[i] * sl2;
-          if (p.soft_cap > 0.f) {
-            const float z = __builtin_amdgcn_exp2f(-fabsf(s[i] * ec));
-            xv = copysignf(p.soft_cap * kLog2e * ((1.f - z) / (1.f + z)), s[i] * sm);
-          }
+          // (tanhf, not a quotient of exponentials: 1 - z loses the score once it is small beside the cap)
+          if (p.soft_cap > 0.f) xv = p.soft_cap * tanhf(s[i] * sm / p.soft_cap) * kLog2e;
           const int kt = key0 + 8 * (i >> 2) + (i & 3);
           const bool masked = kt > st.pos || (p.sliding_window > 0 && kt <= st.pos - p.sliding_window);
           if (masked) xv += p.mask_log2;
@@ -4358,14 +4354,12 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
           if constexpr (has_bias<MODE>()) y[blk][r] += bias[blk][r] * kLog2e;
         }
       if (c >= plain) {
-        if (p.soft_cap > 0.f) {  // soft_cap * tanh(t / soft_cap): sign(t) (1 - z) / (1 + z), z = exp(-2 |t| / soft_cap)
-          const float ec = 2.f * kLog2e / p.soft_cap;
+        if (p.soft_cap > 0.f) {
 #pragma unroll
           for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
             for (int r = 0; r < 4; ++r) {
-              const float t = sc[blk][r] * p.sm_scale, z = __builtin_amdgcn_exp2f(-fabsf(t) * ec);
-              y[blk][r] = copysignf(p.soft_cap * kLog2e * ((1.f - z) / (1.f + z)), t);
+              y[blk][r] = p.soft_cap * tanhf(sc[blk][r] * p.sm_scale / p.soft_cap) * kLog2e;
               if constexpr (has_bias<MODE>()) y[blk][r] += bias[blk][r] * kLog2e;
             }
         }
