@@ -4521,7 +4521,8 @@ bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
   return s->num_tokens <= s->max_num_seqs && cap <= kDirectMaxKeys &&
          cap * (s->head_dim < 64 ? 64 : s->head_dim) <= kDirectElems &&
          (long long)s->max_num_seqs * s->num_kv_heads <= kDirectGroups &&
-         (o->waves_per_cu == 0 || o->waves_per_cu == kMaxWavesPerCU) &&
+         (o->waves_per_cu == 0 || o->waves_per_cu == kMaxWavesPerCU) && o->prefill_tiles == 0 &&
+         o->prefill_cost == 0.f &&
          (unsigned long long)s->total_pages * s->page_size <= 0xffffffffull;  // pool rows in 32 bits
 }
 
