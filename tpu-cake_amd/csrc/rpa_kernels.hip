@@ -4078,14 +4078,22 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
 }
 
 // ---------------------------------------------------------------------------------------------
-// small calls in one launch: one workgroup per (sequence, kv head)
+// small calls in one launch: one workgroup per (block of query rows, kv head)
 // ---------------------------------------------------------------------------------------------
-// A call with at most one query token per sequence slot, short page tables and few (sequence, kv head)
+// A call with no more query tokens than sequence slots, short page tables and few (sequence slot, kv head)
 // pairs is bound by launches and round trips, not by bytes: split over the whole grid it needs a second
 // launch to merge the splits (4.5 us).  Here the eight waves of a workgroup take a sequence's 32-key chunks
 // in turn (wave w: chunks w, w + 8, ...) and merge their (m, l, acc) through LDS.  Two memory round trips:
 // the metadata and the page ids of the wave's first chunks come together (an entry past the sequence's own
 // pages is read, checked and not used), then queries, K and V.
+//
+// A sequence may hold several of the tokens, so workgroups go by token: workgroup (t, h) takes the rows of
+// the 16 / G tokens from t on (one token with G > 16, its rows in blocks of 16) if a block of its sequence
+// starts there.  With one token per sequence, token t is sequence t's; else a workgroup finds its sequence
+// in cu_q_lens, one round trip more.  Consecutive workgroups of an XCD go to its four shader engines in turn,
+// so blocks of four tokens in token order would all land on one of them: each group of four is rotated.
+// One 64-token prompt over 1024 keys in 64 slots, Hq 32 / Hkv 8: 15.9 us (24.2 without the rotation, 156 with
+// a sequence's row blocks one after the other in one workgroup, 56 in the scheduled launches).
 //
 // The same kernel runs the fused decode step (new token, relative bias, cache write: there is no merge
 // launch to store the token) and the v1 contract (separate caches, bias by key position) over its own
@@ -4169,13 +4177,19 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   extern __shared__ __attribute__((aligned(16))) uint8_t smem[];
   float* sml = (float*)(smem + kDirectWaves * kRegion);  // [wave][row][m, l]
   const int lane = threadIdx.x & 63, wv = uni(threadIdx.x >> 6);
-  const int n = lane & 15, j = lane >> 4;
+  int n = lane & 15, j = lane >> 4;
   uint8_t* vt = smem + wv * kRegion;
-  const int i = blockIdx.x / p.Hkv, h = blockIdx.x - i * p.Hkv;
+  int slot = blockIdx.x / p.Hkv;
+  int h = blockIdx.x - slot * p.Hkv;
+  if (slot >> 2 < p.Nmax >> 2) {  // whole groups of four: rotated (see above)
+    const int group = slot >> 2;
+    slot = 4 * group + ((slot + group + (group >> 2)) & 3);
+  }
+  int i = slot;  // the sequence of the workgroup's query rows
   const int D = p.D;
   int err = 0;
 
-  // round trip 1: metadata, page ids of the wave's chunks in [0, kDirectKeys)
+  // round trip 1: metadata and page ids of sequence `slot` (the wave's first two chunks)
   const long long cap = (long long)p.PPS * p.S;
   bool store = true;  // fused: the new token's slot exists
   constexpr bool kV1 = MODE == KV_BF16_BIAS;  // one query token per sequence, no cu_q_lens
@@ -4200,7 +4214,7 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   int nseq = uni(ns_raw);
   nseq = nseq < 0 ? 0 : (nseq > p.Nmax ? p.Nmax : nseq);
   kv = uni(kv);
-  const int q0 = uni(c0);
+  int q0 = uni(c0);
   int ql = kFused ? 1 : uni(c1) - q0;
   bool live = i < nseq;
   if (kv > cap) {
@@ -4214,6 +4228,40 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
     ql = 0;
   }
   if (live && ql > kv) err |= ERR_QLEN;
+  int tok = 0;  // the block's first token in its sequence
+  const int tpb = p.G < ROW_BLOCK ? ROW_BLOCK / p.G : 1;  // tokens of a block
+  if constexpr (!kFused && !kV1) {
+    // the block that starts at token `slot`, if one does.  One token per sequence: sequence `slot`'s, whose
+    // metadata is here; otherwise the token's sequence is looked up
+    if (!(live && q0 <= slot && slot - q0 < ql)) {
+      live = false;
+      if (slot < p.T) {
+#pragma unroll 1
+        for (int s0 = 0; s0 < nseq && !live; s0 += 64) {
+          const int s = s0 + lane < nseq ? s0 + lane : nseq - 1;
+          const int a0 = p.cu_q_lens[s], a1 = p.cu_q_lens[s + 1];
+          const unsigned long long hit = __ballot(a0 >= 0 && a0 <= slot && slot < a1 && a1 <= p.T);
+          if (hit != 0) {
+            const int at = __ffsll(hit) - 1;
+            i = s0 + at;
+            q0 = rl(a0, at);
+            ql = rl(a1, at) - q0;
+            live = true;
+          }
+        }
+      }
+      live = live && (slot - q0) % tpb == 0;
+      if (live) {
+        kv = uni(p.kv_lens[i]);
+        kv = kv > cap ? (int)cap : (kv < 0 ? 0 : kv);
+        prow = (size_t)i * p.PPS;
+        id0 = load_ids(wv);
+        id1 = load_ids(wv + kDirectWaves);
+      }
+    }
+    tok = slot - q0;
+    live = live && tok % tpb == 0;
+  }
   if constexpr (kFused) {  // (make_fused_seq) the sequence's pages start at entry cu_kv / S
     const int cu = uni(c1), pb = page_of(cu, p), npg = kv > 0 ? page(kv - 1) + 1 : 0;
     if (cu < 0 || pb * p.S != cu || (long long)pb + npg > (long long)p.fused_entries) {
@@ -4226,19 +4274,22 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   }
   live = live && ql > 0 && kv > 0;
 
-  const int rows = live ? ql * p.G : 0;
+  // the block's tokens q0 .. q0 + ntok - 1, at key positions pos0 .., and the chunks its rows see
+  const int ntok = kFused || kV1 ? 1 : ql - tok < tpb ? ql - tok : tpb, rows = live ? ntok * p.G : 0;
+  const int pos0 = kv - ql + tok;
+  q0 += tok;
+  const int vis = p.skip_masked && pos0 + ntok < kv ? pos0 + ntok : kv;
+  const int low0 = p.skip_masked && p.sliding_window > 0 ? pos0 - p.sliding_window + 1 : 0;
+  const int first = low0 > 0 ? low0 / KV_CHUNK : 0, last = vis > 0 ? (vis + KV_CHUNK - 1) / KV_CHUNK : 0;
   const bool one_page = p.S % KV_CHUNK == 0;  // a chunk lies in one page
 #pragma unroll 1
-  for (int rb = 0; rb * ROW_BLOCK < rows; ++rb) {
-    const int nch = rb_units(kv, ql, p.G, rb, p.skip_masked, p.sliding_window);
-    const int first = rb_first_chunk(kv, ql, p.G, rb, p.skip_masked, p.sliding_window);
-    if (nch == 0) continue;
-    const int last = first + nch;
+  for (int rb = 0; rb * ROW_BLOCK < rows && first < last; ++rb) {  // (more than one turn: G > 16, one token)
+    asm volatile("" : "+s"(kv), "+s"(h), "+s"(i), "+v"(n), "+v"(j));  // (nothing of a turn is kept in registers for the next)
     // the wave's chunks of this block: those of its residue class from `first` on
     const int row = rb * ROW_BLOCK + n, rrow = row < rows ? row : 0;
-    const int tok = rrow / p.G, g = rrow - tok * p.G;
-    const int pos = kv - ql + (row < rows ? tok : 0);
-    const size_t qrow = (size_t)(q0 + tok) * p.Hq + (size_t)h * p.G + g;
+    const int rtok = kFused || kV1 ? 0 : rrow / p.G, g = rrow - rtok * p.G;
+    const int pos = pos0 + (row < rows ? rtok : 0);
+    const size_t qrow = (size_t)(q0 + rtok) * p.Hq + (size_t)h * p.G + g;
     bf16x8 q[KS];
     uint2 rst = {0u, 0u};
 #pragma unroll
@@ -4257,7 +4308,6 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
     const uint8_t* kbase = a.kb + (size_t)h * a.head;
     const uint8_t* vbase = a.vb + (size_t)h * a.head;
     // chunks that every row sees in full, without a soft cap or a window, skip the masks
-    const int pos0 = kv - ql + rb * ROW_BLOCK / p.G;
     const int plain = p.soft_cap > 0.f || p.sliding_window > 0 ? 0 : ((pos0 + 1 < kv ? pos0 + 1 : kv) / KV_CHUNK);
     using Half = DirectHalf<MODE, DW>;
     const int piece = 16 * (lane % Half::kLanes);  // (pieces wholly past D read the row's first piece)
@@ -4514,8 +4564,8 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   RPA_TL(tl_set(TL_END, tl_clock());)
 }
 
-// Whether a call runs as one workgroup per (sequence, kv head) in a single launch (bounds: see the
-// kernel), with no schedule knob asked for.
+// Whether a call runs as one workgroup per (block of query rows, kv head) in a single launch (bounds: see
+// the kernel), with no schedule knob asked for.
 bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
   const long long cap = (long long)s->pages_per_seq * s->page_size;
   return s->num_tokens <= s->max_num_seqs && cap <= kDirectMaxKeys &&

@@ -346,7 +346,7 @@ DIRECT_ELEMS, DIRECT_GROUPS, DIRECT_MAX_KEYS, DIRECT_WAVES = 1024 * 128, 512, 40
 
 
 def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, table_keys: int) -> bool:
-    """Whether a call runs in one launch, a workgroup per (sequence, kv head) (direct_call with the
+    """Whether a call runs in one launch, a workgroup per (block of query rows, kv head) (direct_call with the
     default knobs); table_keys: the keys a sequence's page table holds."""
     return (num_tokens <= max_num_seqs and table_keys <= DIRECT_MAX_KEYS
             and table_keys * max(head_dim, 64) <= DIRECT_ELEMS and max_num_seqs * hkv <= DIRECT_GROUPS)
@@ -354,7 +354,7 @@ def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, tab
 
 def _direct_line(seqs: int, hkv: int, what: str) -> str:
     return (f"launch (short page tables) = rpa_attn_kernel_direct: grid {seqs * hkv} x block {64 * DIRECT_WAVES} (one "
-            f"workgroup per (sequence, kv head), its waves' states merged in LDS; {what}); longer page tables or more "
+            f"workgroup per (block of query rows, kv head), its waves' states merged in LDS; {what}); longer page tables or more "
             "pairs take the launches below")
 
 
