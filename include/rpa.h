@@ -86,10 +86,10 @@ typedef struct rpa_shape {
  *                  units, which sets the work split between the two roles
  *                  (0 = 0.45).
  * With all three at their defaults (waves_per_cu 0 or 8), a small call -- num_tokens <=
- * max_num_seqs, pages_per_seq * page_size <= 4096 keys and times max(head_dim, 64) <= 2^17,
- * max_num_seqs * num_kv_heads <= 512 -- is one launch of its own kernel, with no roles to
- * schedule; a nonzero prefill_tiles or prefill_cost, or a waves_per_cu cap, keeps the launches
- * those knobs describe. */
+ * max_num_seqs, at most 512 (sequence slot, kv head) pairs, short page tables (1024 keys of 128
+ * dims; fewer with more than 256 pairs or more than 16 query heads per kv head) -- is one launch
+ * of its own kernel, with no roles to schedule; a nonzero prefill_tiles or prefill_cost, or a
+ * waves_per_cu cap, keeps the launches those knobs describe. */
 typedef struct rpa_options {
   float sm_scale;
   int32_t sliding_window;

@@ -15,7 +15,7 @@ def library():
         build.build()
 
 
-def _case(tokens=64, slots=64, g=4, hkv=8, dim=128, page=64, keys=1024, dtype="bf16"):
+def _case(tokens=60, slots=60, g=4, hkv=4, dim=128, page=64, keys=1024, dtype="bf16"):
     shape = lambda *s: np.empty(s, np.uint8)  # noqa: E731
     return types.SimpleNamespace(q=shape(tokens, hkv * g, dim), kv_pages=shape(2, page, 2 * hkv, dim),
                                  page_indices=shape(slots, -(-keys // page)), kv_dtype=dtype, sm_scale=1.0)
@@ -23,7 +23,7 @@ def _case(tokens=64, slots=64, g=4, hkv=8, dim=128, page=64, keys=1024, dtype="b
 
 def _direct(case, knobs=None):
     slots, hkv = case.page_indices.shape[0], case.kv_pages.shape[2] // 2
-    return ops.attention_grid(case, knobs, cus=256) == (slots * hkv, 8) and slots * hkv != 256
+    return ops.attention_grid(case, knobs, cus=256) == (slots * hkv, 8)
 
 
 @pytest.mark.parametrize("dtype", ["bf16", "fp8"])
@@ -36,11 +36,25 @@ def test_schedule_knobs_keep_their_launches(dtype, knobs, direct):
 
 
 @pytest.mark.parametrize("kw,direct", [
-    ({}, True), (dict(tokens=65), False), (dict(keys=1025), False), (dict(dim=64, keys=2048), True),
+    ({}, True), (dict(tokens=61), False), (dict(keys=1025), False), (dict(dim=64, keys=2048), True),
     (dict(dim=32, keys=2049), False), (dict(dim=256, keys=512), True), (dict(dim=256, keys=513), False),
-    (dict(slots=65, tokens=1), False), (dict(slots=512, tokens=512, hkv=1), True), (dict(page=20, keys=1020), True)])
+    (dict(page=20, keys=1020), True),
+    # more pairs than CUs: a second round of workgroups
+    (dict(slots=65), False), (dict(slots=65, keys=512), True), (dict(slots=128, keys=513), False),
+    (dict(slots=129, keys=64), False), (dict(slots=65, keys=512, dtype="fp8"), False),
+    (dict(slots=65, keys=256, dtype="fp8"), True), (dict(slots=128, dim=64, keys=2048, dtype="fp8"), True),
+    (dict(slots=65, dim=256, keys=128), False), (dict(slots=65, dim=256, keys=64), True),
+    (dict(slots=65, dim=256, keys=512, dtype="fp8"), True), (dict(slots=65, dim=32, keys=2048), True),
+    (dict(slots=65, dim=64, keys=1088), False),
+    # more than 16 query heads per kv head: several turns over the same keys
+    (dict(slots=4, tokens=4, hkv=1, g=32), False), (dict(slots=4, tokens=4, hkv=1, g=32, keys=512), True),
+    (dict(slots=14, tokens=14, hkv=1, g=32), True), (dict(slots=4, tokens=4, hkv=1, g=64, keys=256), False),
+    (dict(slots=4, tokens=4, hkv=1, g=64, keys=128), True), (dict(hkv=1, g=64, keys=512), True),
+    (dict(hkv=1, g=65, keys=64), False), (dict(slots=128, g=32, keys=192), False),
+    (dict(slots=128, g=32, keys=128), True)])
 def test_bounds(kw, direct):
     case = _case(**kw)
     assert _direct(case) == direct
     hkv, table = case.kv_pages.shape[2] // 2, case.page_indices.shape[1] * case.kv_pages.shape[1]
-    assert contracts.direct_call(case.q.shape[0], case.page_indices.shape[0], hkv, case.q.shape[2], table) == direct
+    assert contracts.direct_call(case.q.shape[0], case.page_indices.shape[0], hkv, case.q.shape[2], table,
+                                 case.q.shape[1] // hkv, case.kv_dtype) == direct

@@ -4101,13 +4101,10 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
 //
 // Per call in a captured step, 4 sequences, Hq 8 / Hkv 2, page 16, D 128 (before: split and merged): 32 keys
 // 7.9 -> 4.3 us, 128 keys 10.0 -> 5.2, 512 keys 11.1 -> 8.8; 32 sequences of 512 keys at Hq 32 / Hkv 8
-// 26.1 -> 17.9.  The rule's bounds (direct_call): one CU reads a pair's K and V, so past kDirectElems
-// elements of K the split form is ahead (bf16, D 128, lengths uniform up to the table's end: 1024 keys 1.2 to
-// 1.5x faster here, 2048 keys 0.83 to 1.25x; D 64 still 1.4 to 2.2x at 2048, D 256 0.8 to 1.1x at 1024), and
-// past kDirectGroups pairs the grid is full either way (1024 pairs: bf16 1.07x, fp8 0.8x).
+// 23.8 -> 18.1.  Bounds of the rule: direct_fits.
 constexpr int kDirectWaves = 8;
 constexpr int kDirectElems = 1024 * 128;  // keys of a page table x row width
-constexpr int kDirectGroups = 512;        // sequence slots x kv heads: two workgroups per CU
+constexpr int kDirectPairs = 256;         // (sequence slot, kv head) pairs of one round: a workgroup fills a CU
 constexpr int kDirectMaxKeys = 4096;      // (pmagic's range)
 
 struct DirectArgs {
@@ -4564,13 +4561,43 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   RPA_TL(tl_set(TL_END, tl_clock());)
 }
 
-// Whether a call runs as one workgroup per (block of query rows, kv head) in a single launch (bounds: see
-// the kernel), with no schedule knob asked for.
+// Whether the one-launch kernel is ahead of the scheduled launches for page tables of cap keys, D-dim heads, G
+// query heads per kv head and `pairs` (sequence slot, kv head) pairs.  One CU reads a pair's K and V, its
+// workgroup fills the CU, and a pair's rows past 16 take further turns over the same keys.  us per captured call,
+// scheduled / here, lengths uniform up to the table's end and all at it (bf16, D 128 unless said):
+//   G <= 16, pairs <= 256: to 1024 x 128 elements per pair.  256 pairs of 1024 keys 27.3 / 22.8, 34.0 / 30.1;
+//     fp8 22.4 / 18.1, 25.1 / 21.4; D 64, 2048 keys 25.4 / 22.8, 33.0 / 29.2; D 256, 512 keys 29.5 / 28.1,
+//     36.0 / 36.7.  (Of 2048 keys 0.83 to 1.25x.)
+//   G <= 16, a second round, 320 to 512 pairs, to a share of those elements that depends on how far the scheduled
+//     launches are ahead by then: bf16 to one half (512 keys 22.4 / 16.1 to 34.2 / 33.9; 1024 keys 27.7 / 27.1,
+//     40.3 / 44.3), D < 64 to all (2048 keys 22.4 / 17.6 to 41.8 / 34.3), D 256 to one eighth (64 keys 16.6 / 13.6
+//     to 22.5 / 19.6; 128 keys 18.2 / 15.3 to 26.4 / 29.6); fp8 to one quarter (256 keys 14.6 / 12.4 to 19.1 / 17.0;
+//     512 keys 19.1 / 14.9 to 25.5 / 27.3), D <= 64 or 256 to all (D 64, 2048 keys 33.3 / 20.4 to 70.3 / 38.6).
+//   G 17 to 64, t = 2 to 4 turns: to 2^(1-t) of the elements, which few pairs do not lose (4 pairs: G 32, 512 keys
+//     19.6 / 15.1, 1024 keys 23.3 / 21.3, 14.3 / 21.9; G 48, 256 keys 17.2 / 15.1; G 64, 128 keys 16.3 / 15.0, 512
+//     keys 20.3 / 27.5), to 3 / t of them from 7 t pairs on (G 32, 14 pairs of 1024 keys 24.2 / 19.8, 20.1 / 22.4;
+//     G 48, 24 pairs 31.4 / 28.1; G 64, 48 pairs of 512 keys 30.0 / 28.6, 40.1 / 29.0); a second round to 1 / 4 t
+//     (G 32, 512 pairs of 128 keys 41.7 / 18.2).
+//   G > 64: never (G 128, 64 keys 17.3 / 22.4; 1024 keys 30.1 / 76.9).
+bool direct_fits(long long cap, int D, bool fp8, int G, long long pairs) {
+  const long long elems = cap * (D < 64 ? 64 : D);
+  const int turns = (G + ROW_BLOCK - 1) / ROW_BLOCK;
+  if (cap > kDirectMaxKeys || elems > kDirectElems || pairs > 2 * kDirectPairs || turns > 4) return false;
+  if (pairs > kDirectPairs) {
+    const bool wide = D > 64 && D <= 128;
+    const int share = fp8 ? (wide ? 4 : 1) : D < 64 ? 1 : D <= 128 ? 2 : 8;
+    return elems <= kDirectElems / share && (turns == 1 || elems * turns <= kDirectElems / 4);
+  }
+  return turns == 1 || elems << (turns - 1) <= kDirectElems ||
+         (pairs >= 7 * turns && elems * turns <= 3 * kDirectElems);
+}
+
+// Whether a call runs as one workgroup per (block of query rows, kv head) in a single launch, with no schedule
+// knob asked for.
 bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
-  const long long cap = (long long)s->pages_per_seq * s->page_size;
-  return s->num_tokens <= s->max_num_seqs && cap <= kDirectMaxKeys &&
-         cap * (s->head_dim < 64 ? 64 : s->head_dim) <= kDirectElems &&
-         (long long)s->max_num_seqs * s->num_kv_heads <= kDirectGroups &&
+  return s->num_tokens <= s->max_num_seqs &&
+         direct_fits((long long)s->pages_per_seq * s->page_size, s->head_dim, s->kv_dtype == RPA_KV_FP8_E4M3,
+                     s->num_q_heads / s->num_kv_heads, (long long)s->max_num_seqs * s->num_kv_heads) &&
          (o->waves_per_cu == 0 || o->waves_per_cu == kMaxWavesPerCU) && o->prefill_tiles == 0 &&
          o->prefill_cost == 0.f &&
          (unsigned long long)s->total_pages * s->page_size <= 0xffffffffull;  // pool rows in 32 bits

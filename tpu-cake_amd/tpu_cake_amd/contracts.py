@@ -342,14 +342,25 @@ def _work_split(kv_lens, q_lens, hq: int, hkv: int, kv_dtype: str, prefill_tiles
                 prefill_chunk_steps=round(steps))
 
 
-DIRECT_ELEMS, DIRECT_GROUPS, DIRECT_MAX_KEYS, DIRECT_WAVES = 1024 * 128, 512, 4096, 8  # csrc/rpa_kernels.hip, direct_call
+DIRECT_ELEMS, DIRECT_PAIRS, DIRECT_MAX_KEYS, DIRECT_WAVES = 1024 * 128, 256, 4096, 8  # csrc/rpa_kernels.hip, direct_fits
 
 
-def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, table_keys: int) -> bool:
+def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, table_keys: int, group: int = 1,
+                kv_dtype: str = "bf16") -> bool:
     """Whether a call runs in one launch, a workgroup per (block of query rows, kv head) (direct_call with the
-    default knobs); table_keys: the keys a sequence's page table holds."""
-    return (num_tokens <= max_num_seqs and table_keys <= DIRECT_MAX_KEYS
-            and table_keys * max(head_dim, 64) <= DIRECT_ELEMS and max_num_seqs * hkv <= DIRECT_GROUPS)
+    default knobs; the reasons are at direct_fits); table_keys: the keys a sequence's page table holds."""
+    elems, turns, pairs = table_keys * max(head_dim, 64), -(-group // 16), max_num_seqs * hkv
+    if (num_tokens > max_num_seqs or table_keys > DIRECT_MAX_KEYS or elems > DIRECT_ELEMS or pairs > 2 * DIRECT_PAIRS
+            or turns > 4):
+        return False
+    if pairs > DIRECT_PAIRS:
+        if kv_dtype == "fp8":
+            share = 4 if 64 < head_dim <= 128 else 1
+        else:
+            share = 1 if head_dim < 64 else 2 if head_dim <= 128 else 8
+        return elems <= DIRECT_ELEMS // share and (turns == 1 or elems * turns <= DIRECT_ELEMS // 4)
+    return (turns == 1 or elems << (turns - 1) <= DIRECT_ELEMS
+            or (pairs >= 7 * turns and elems * turns <= 3 * DIRECT_ELEMS))
 
 
 def _direct_line(seqs: int, hkv: int, what: str) -> str:
@@ -406,7 +417,8 @@ def _operator_workload(cfg: str) -> tuple[str, WorkloadContract, dict]:
     floor_mfma = fl["mfma_s"] * 1e6
     half = split["grid"] // 2
     fixed = co and split["prefill_workgroups"] == half and half % 8 == 0
-    direct = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size)
+    direct = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size,
+                         m.num_q_heads // m.num_kv_heads, m.kv_dtype)
     lines = [
         f"description = {CONFIG_DESCRIPTIONS[cfg]}",
         "entry = rpa_ragged_paged_attention (include/rpa.h); one call = the two launches below, stream-ordered",

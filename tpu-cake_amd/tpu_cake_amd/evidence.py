@@ -136,7 +136,8 @@ def call_kernels(config: str) -> tuple:
     from .workloads import make_config_meta_for
 
     m, _ = make_config_meta_for(config)
-    small = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size)
+    small = direct_call(m.num_tokens, m.num_seqs, m.num_kv_heads, m.head_dim, m.pages_per_seq * m.page_size,
+                         m.num_q_heads // m.num_kv_heads, m.kv_dtype)
     return KERNELS[:1] if small else KERNELS
 
 
