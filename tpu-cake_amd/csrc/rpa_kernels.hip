@@ -4592,6 +4592,23 @@ bool direct_fits(long long cap, int D, bool fp8, int G, long long pairs) {
          (pairs >= 7 * turns && elems * turns <= 3 * kDirectElems);
 }
 
+// The same for the v1 contract.  Its other form packs both caches, whole, on every call, so this one is ahead
+// further: past direct_fits while 4 us and, per turn and round, 2 us and 9 per kDirectElems elements come to less
+// than 14 us and the packed caches at 2 MiB a us.  us per captured call, packed / here, lengths uniform and full,
+// 4096 keys, D 128: 1 sequence of 1 kv head, G 8 13.7 / 24.6, 15.8 / 43.4; of 8 kv heads, G 4 23.2 / 24.0,
+// 27.3 / 42.2; 4 of 8 49.0 / 40.5, 49.4 / 50.0; 16 of 8 139 / 59, 158 / 76; 64 of 8 581 / 155, 671 / 214; 1024 keys
+// of 64 dims: 4 of 1, G 64 28.5 / 45.2, 20.3 / 46.3; 256 of 8, G 1 459 / 85, 551 / 129.
+bool v1_direct_fits(const rpa_inkling_shape_t* f) {
+  const long long cap = (long long)f->pages_per_seq * f->page_size, pairs = (long long)f->num_seqs * f->num_kv_heads;
+  const int G = f->num_q_heads / f->num_kv_heads;
+  if (cap > kDirectMaxKeys) return false;
+  if (direct_fits(cap, f->head_dim, false, G, pairs)) return true;
+  const double elems = (double)cap * (f->head_dim < 64 ? 64 : f->head_dim);
+  const double turns = (double)((pairs + kDirectPairs - 1) / kDirectPairs) * ((G + ROW_BLOCK - 1) / ROW_BLOCK);
+  const double packed = (double)f->total_pages * f->page_size * 2 * f->num_kv_heads * kD * 2;
+  return 4 + turns * (2 + 9 * elems / kDirectElems) <= 14 + packed / (1 << 21);
+}
+
 // Whether a call runs as one workgroup per (block of query rows, kv head) in a single launch, with no schedule
 // knob asked for.
 bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
@@ -5733,8 +5750,7 @@ int rpa_inkling_decode(const rpa_inkling_shape_t* f, float sm_scale, const void*
   a.L = f->bias_len;
   a.vec = ((uintptr_t)key_cache | (uintptr_t)value_cache) % 16 == 0 && a.D % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
-  if (a.vec && (long long)f->pages_per_seq * f->page_size <= kDirectMaxKeys &&
-      (unsigned long long)f->total_pages * f->page_size <= 0xffffffffull) {
+  if (a.vec && v1_direct_fits(f) && (unsigned long long)f->total_pages * f->page_size <= 0xffffffffull) {
     // one launch over the caller's own caches (nothing packed, padded or merged)
     const rpa_shape_t ds = v1_rpa_shape(f);
     Params p = base_params(&ds);
