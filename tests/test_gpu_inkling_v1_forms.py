@@ -102,3 +102,15 @@ def test_a_cache_off_the_16_byte_grid(cuda, which):
     out = inkling.inkling_rpa(*args)
     assert _max_abs(out, host) <= TOL
     assert _call(args)[2]
+
+
+def test_out_may_alias_the_query_below_128_dims_only(cuda):
+    print("[case] out is the query", flush=True)
+    for keys, packed in ((256, False), (4112, True)):
+        host = _inputs([7, 64, 200], 8, 4, 64, 16, keys, 4)
+        args = _device(host)
+        rc, out, did_pack = _call(args, out=args[0])
+        assert rc == 0 and did_pack == packed
+        assert _max_abs(out, host) <= TOL
+        wide = _device(_inputs([7, 64, 200], 8, 4, 128, 16, keys, 5))
+        assert _call(wide, out=wide[0])[0] == -1  # RPA_E_INVALID

@@ -5723,6 +5723,8 @@ int rpa_inkling_decode(const rpa_inkling_shape_t* f, float sm_scale, const void*
   if (rc) return rc;
   if (!query || !key_cache || !value_cache || !page_table || !sequence_lengths || !bias || !out)
     return fail(RPA_E_INVALID, "inkling: NULL pointer");
+  // (a narrower head dim may alias: either form has read a row's queries before it writes the row)
+  if (query == out && f->head_dim == kD) return fail(RPA_E_INVALID, "out must not alias q");
   DeviceInfo d;
   rc = device_info(d);
   if (rc) return rc;
