@@ -91,17 +91,20 @@ def test_forms(cuda, lengths, hq, hkv, d, page, keys, packed):
     assert did_pack == packed
 
 
-@pytest.mark.parametrize("which", [1, 2])
-def test_a_cache_off_the_16_byte_grid(cuda, which):
-    print(f"[case] cache {which} at an odd address", flush=True)
-    host = _inputs([7, 64, 200], 8, 4, 64, 16, 256, 3)
+@pytest.mark.parametrize("d,which", [(64, 0), (64, 1), (64, 2), (64, 6), (128, 0), (128, 6), (32, 6)])
+def test_tensors_off_their_alignment(cuda, d, which):
+    # 0 the query, 1 and 2 the caches, 6 the output, one element past a 16-byte boundary: the packed form
+    print(f"[case] D {d} tensor {which} at an odd address", flush=True)
+    host = _inputs([7, 64, 200], 8, 4, d, 16, 256, 3)
     args = _device(host)
+    args.append(torch.empty_like(args[0]))
     flat = torch.empty(args[which].numel() + 1, dtype=torch.bfloat16, device="cuda")
     flat[1:] = args[which].flatten()
     args[which] = flat[1:].view(args[which].shape)
-    out = inkling.inkling_rpa(*args)
+    rc, out, did_pack = _call(args[:6], out=args[6])
+    assert rc == 0 and did_pack
     assert _max_abs(out, host) <= TOL
-    assert _call(args)[2]
+    assert _max_abs(inkling.inkling_rpa(*args[:6], out=args[6]), host) <= TOL
 
 
 def test_out_may_alias_the_query_below_128_dims_only(cuda):

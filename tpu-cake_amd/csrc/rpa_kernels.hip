@@ -5752,7 +5752,9 @@ int rpa_inkling_decode(const rpa_inkling_shape_t* f, float sm_scale, const void*
   a.L = f->bias_len;
   a.vec = ((uintptr_t)key_cache | (uintptr_t)value_cache) % 16 == 0 && a.D % 8 == 0;
   hipStream_t st = (hipStream_t)stream;
-  if (a.vec && v1_direct_fits(f) && (unsigned long long)f->total_pages * f->page_size <= 0xffffffffull) {
+  // the one-launch form reads queries 16 bytes and writes rows 8 bytes at a time (packing goes by element)
+  const bool io = (uintptr_t)query % 16 == 0 && (uintptr_t)out % 8 == 0;
+  if (a.vec && io && v1_direct_fits(f) && (unsigned long long)f->total_pages * f->page_size <= 0xffffffffull) {
     // one launch over the caller's own caches (nothing packed, padded or merged)
     const rpa_shape_t ds = v1_rpa_shape(f);
     Params p = base_params(&ds);
