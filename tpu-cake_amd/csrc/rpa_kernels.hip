@@ -4261,7 +4261,8 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   }
   if constexpr (kFused) {  // (make_fused_seq) the sequence's pages start at entry cu_kv / S
     const int cu = uni(c1), pb = page_of(cu, p), npg = kv > 0 ? page(kv - 1) + 1 : 0;
-    if (cu < 0 || pb * p.S != cu || (long long)pb + npg > (long long)p.fused_entries) {
+    // (no new token: nowhere to store it)
+    if (cu < 0 || pb * p.S != cu || (long long)pb + npg > (long long)p.fused_entries || kv < 1) {
       if (live) err |= ERR_PAGE;
       live = false;
     }
