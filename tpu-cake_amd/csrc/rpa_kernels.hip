@@ -2198,9 +2198,10 @@ struct CoSeg {
   int c_lo, c_hi;  // chunks
 };
 
-// A row's running maximum before its first visible key: below every score, and finite, so that the
-// exponent of a masked score (-inf) and the first rescale (2^(start - m) = 0) need no special case.
-constexpr float kMaxStart = -1e30f;
+// A row's running maximum before its first visible key: no score is below it, and it is finite, so that the
+// exponent of a masked score (-inf) and the first rescale (2^(start - m) = 0, or 1 over zeros) need no special
+// case.
+constexpr float kMaxStart = -3.402823466e38f;
 
 // The rows of one 32-row block: row = lane % 32; acc element v of block db is dim
 // 32 db + 8 (v / 4) + 4 (lane / 32) + v % 4; l sums the lane's own 16 keys of each chunk.
