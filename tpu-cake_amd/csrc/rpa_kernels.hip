@@ -2071,19 +2071,20 @@ constexpr bool co_converts() {  // a pass per step (scaled or fp8)
   return MODE != KV_BF16;
 }
 
-// LDS geometry of a chunk of DT-wide key rows (DT 64, 128 or 256; narrower heads are padded to one).
+// LDS geometry of a chunk of DT-wide key rows.
 template <int DT>
 struct CoGeo {
+  static_assert(DT == 64 || DT == 128, "tiles of 64- and 128-dim heads");
   static constexpr int kRow = 2 * DT;              // bytes of a key row
   static constexpr int kBlkKeys = 1024 / kRow;     // keys per KiB block (one DMA)
   static constexpr int kBlks = KV_CHUNK / kBlkKeys;
-  static constexpr int kKPad = DT == 256 ? 32 : 64, kVPad = DT == 256 ? 128 : 0;
-  static constexpr int kKBlk = 1024 + kKPad, kVBlk = 1024 + kVPad;
+  static constexpr int kKPad = 64;
+  static constexpr int kKBlk = 1024 + kKPad, kVBlk = 1024;
   static constexpr int kKSlot = kBlks * kKBlk, kVSlot = kBlks * kVBlk;
   static constexpr int kSteps = DT / 16;           // QK^T k-steps of 16 dims
   static constexpr int kDb = DT / 32;              // PV dim blocks of 32
-  static __device__ __forceinline__ int xk(int key) { return DT == 64 ? (key >> 1) & 3 : DT == 128 ? key & 3 : key & 1; }
-  static __device__ __forceinline__ int xv(int key) { return DT == 64 ? (key >> 1) & 1 : DT == 128 ? key & 3 : key & 1; }
+  static __device__ __forceinline__ int xk(int key) { return DT == 64 ? (key >> 1) & 3 : key & 3; }
+  static __device__ __forceinline__ int xv(int key) { return DT == 64 ? (key >> 1) & 1 : key & 3; }
 };
 
 template <int MODE, int DT, bool UPG>
@@ -2106,7 +2107,7 @@ struct CoLds {
   static constexpr int kBytes = kFlags + kCoWaves * 4;
   // DMAs per wave and step: kPerOp per operand; with fp8 rows of 64 bytes a wave carries one operand
   static constexpr bool kOneOp = kFp8 && DT == 64;
-  static constexpr int kPerOp = kFp8 ? (DT >= 128 ? DT / 128 : 1) : Geo::kBlks / kCoWaves;
+  static constexpr int kPerOp = kFp8 ? 1 : Geo::kBlks / kCoWaves;
   static constexpr int kStepDmas = kOneOp ? 1 : 2 * kPerOp;
 };
 
@@ -2118,9 +2119,6 @@ __device__ __forceinline__ void co_barrier() {
   static_assert(N >= 0 && N < 64, "co_barrier's vmcnt");
   asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" : : "n"(N) : "memory");
 }
-
-// Every DMA of this wave has landed.
-__device__ __forceinline__ void co_drain() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 
 // Byte address in LDS of a pointer into the workgroup's LDS.
 __device__ __forceinline__ uint32_t lds_addr_of(const void* ptr) {
@@ -2152,14 +2150,12 @@ __device__ __forceinline__ void co_dma_s(const void* base, uint32_t off, uint32_
 
 // A workgroup's chunk loads, the same for every tile: DMA t of this wave carries key key(t) of the
 // chunk, bytes colk(t) of its K row and colv(t) of its V row (from the first byte of the key's K row).
-// A narrow row's pieces wholly past D read the row's first piece (zero query dims, unstored outputs).
 template <int MODE, int DT, bool UPG>
 struct CoLoads {
   using L = CoLds<MODE, DT, UPG>;
   using Geo = CoGeo<DT>;
   int wv, lane;
   uint32_t row;              // bytes between consecutive keys of a page
-  int D;
   uint32_t offk[L::kPerOp], offv[L::kPerOp];  // key(t) * row + colk(t) / colv(t)
   uint32_t offt[L::kPerOp];                   // offv with keys past the current tile's last one read as it
 
@@ -2168,12 +2164,11 @@ struct CoLoads {
     constexpr int kKeys = L::kFp8 ? 1024 / DT : Geo::kBlkKeys;
     return blk(t) * kKeys + lane / (64 / kKeys);
   }
-  __device__ __forceinline__ void init(const Params& p, int D_, int wv_, int lane_) {
+  __device__ __forceinline__ void init(const Params& p, int wv_, int lane_) {
     wv = wv_;
     lane = lane_;
-    D = D_;
     constexpr int kElem = L::kFp8 ? 1 : 2;
-    row = (uint32_t)(2 * p.Hkv) * D * kElem;
+    row = (uint32_t)(2 * p.Hkv) * DT * kElem;
 #pragma unroll
     for (int t = 0; t < L::kPerOp; ++t) {
       const int k = key(t);
@@ -2185,10 +2180,8 @@ struct CoLoads {
         ck = 8 * (pos ^ Geo::xk(k));
         cv = 32 * ((pos >> 2) ^ Geo::xv(k)) + 8 * (pos & 3);
       }
-      ck = ck < D ? ck : 0;
-      cv = cv < D ? cv : 0;
       offk[t] = (uint32_t)k * row + ck * kElem;
-      offv[t] = (uint32_t)k * row + (D + cv) * kElem;
+      offv[t] = (uint32_t)k * row + (DT + cv) * kElem;
     }
   }
 };
@@ -2244,8 +2237,8 @@ struct CoTile {
   int c_tail;                      // the chunk with keys past kv_len (-1: none)
   int plain_to;                    // chunks below it need no masking
   typedef __attribute__((address_space(3))) const uint8_t* lds_cp;
-  lds_cp kfrag[DT == 256 ? 1 : 2];  // this lane's A fragments in K slot 0 (k-steps 0 and 1)
-  lds_cp vfrag[DT == 256 ? 2 : Geo::kDb];  // its transposing reads in V slot 0 by dim block
+  lds_cp kfrag[2];                  // this lane's A fragments in K slot 0 (k-steps 0 and 1)
+  lds_cp vfrag[Geo::kDb];           // its transposing reads in V slot 0 by dim block
   uint32_t dstk, dstv;              // LDS addresses of this wave's first DMA block of ring slot 0
 
   static constexpr int kAhead = L::kFp8 ? 1 : 0;  // fp8 chunks are issued one step further ahead
@@ -2277,7 +2270,7 @@ struct CoTile {
         co_dma_s(base, v ? (c == c_tail ? ld.offt[t] : ld.offv[t]) : ld.offk[t], dst, imm);
       } else {
         const uint32_t col = (v ? ld.offv[t] : ld.offk[t]) - (uint32_t)ld.key(t) * ld.row;
-        co_dma(p.kv + (size_t)rows[t] * ld.row + (size_t)(2 * tl.h) * ld.D * (L::kFp8 ? 1 : 2) + col, dst, imm);
+        co_dma(p.kv + (size_t)rows[t] * ld.row + (size_t)(2 * tl.h) * DT * (L::kFp8 ? 1 : 2) + col, dst, imm);
       }
     }
   }
@@ -2355,14 +2348,13 @@ struct CoTile {
 
   __device__ __forceinline__ bf16x8 k_fragment(int rel, int s) const {
     typedef __attribute__((address_space(3))) const bf16x8* lds_b8;
-    if constexpr (DT == 256) return *(lds_b8)(kfrag[0] + slot_at(rel, false) + 32 * s);
     return *(lds_b8)(kfrag[s & 1] + slot_at(rel, false) + 64 * (s >> 1));
   }
   __device__ __forceinline__ bf16x8 v_fragment(int rel, int db, int t) const {
     typedef __attribute__((address_space(3))) short4_t* lds_s4;
     // keys 16t + 8 lh + ..: whole blocks further
     constexpr int kStep = (8 / Geo::kBlkKeys) * Geo::kVBlk;
-    const lds_cp b = (DT == 256 ? vfrag[db & 1] + 128 * (db >> 1) : vfrag[db]) + slot_at(rel, true) + 2 * t * kStep;
+    const lds_cp b = vfrag[db] + slot_at(rel, true) + 2 * t * kStep;
     const short4_t lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)b);
     const short4_t hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s4)(b + kStep));
     return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, hi, 0, 1, 2, 3, 4, 5, 6, 7));
@@ -2371,18 +2363,14 @@ struct CoTile {
     n32 = lane & 31;
     hf = lane >> 5;
     const lds_cp kr = (lds_cp)(lds + L::kK) + (n32 / Geo::kBlkKeys) * Geo::kKBlk + (n32 % Geo::kBlkKeys) * Geo::kRow;
-    if constexpr (DT == 256) {
-      kfrag[0] = kr + 16 * (hf ^ Geo::xk(n32));
-    } else {
-      kfrag[0] = kr + 16 * (hf ^ Geo::xk(n32));
-      kfrag[1] = kr + 16 * ((2 + hf) ^ Geo::xk(n32));
-    }
+    kfrag[0] = kr + 16 * (hf ^ Geo::xk(n32));
+    kfrag[1] = kr + 16 * ((2 + hf) ^ Geo::xk(n32));
     // lane nn of group (hf, dsub) addresses key 4 hf + nn / 4, dims 16 dsub + 4 (nn % 4) .. of a block
     const int nn = lane & 15, dsub = (lane >> 4) & 1, k0 = 4 * hf + (nn >> 2);
     const lds_cp vr = (lds_cp)(lds + L::kV) + (k0 / Geo::kBlkKeys) * Geo::kVBlk + (k0 % Geo::kBlkKeys) * Geo::kRow +
                       32 * dsub + 8 * (nn & 3);
 #pragma unroll
-    for (int d = 0; d < (DT == 256 ? 2 : Geo::kDb); ++d) vfrag[d] = vr + 64 * (d ^ Geo::xv(k0));
+    for (int d = 0; d < Geo::kDb; ++d) vfrag[d] = vr + 64 * (d ^ Geo::xv(k0));
     const int w = ld.blk(0);
     dstk = uni((int)(lds_addr_of(lds + (L::kFp8 ? 0 : L::kK)) + (uint32_t)w * (L::kFp8 ? 1024 : Geo::kKBlk)));
     dstv = uni((int)(lds_addr_of(lds + (L::kFp8 ? L::kCodeV : L::kV)) + (uint32_t)w * (L::kFp8 ? 1024 : Geo::kVBlk)));
@@ -2559,7 +2547,7 @@ struct CoTile {
         pg = 0;
       }
       if constexpr (UPG)
-        ((uint64_t*)tab)[t] = kv_elem(p, pg, kt, 2 * tl.h, ld.D) * (L::kFp8 ? 1 : 2);
+        ((uint64_t*)tab)[t] = kv_elem(p, pg, kt, 2 * tl.h, DT) * (L::kFp8 ? 1 : 2);
       else
         tab[t] = (uint32_t)pg * (uint32_t)p.S + (uint32_t)slot_of(kt, p);
       if constexpr (L::kFp8) {  // the page's K and V scales of kv head h
@@ -2647,7 +2635,6 @@ __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoa
                                         uint8_t* lds, int wv, int lane, int& err, int slot, TlAcc& ta) {
   using L = CoLds<MODE, DT, UPG>;
   using Geo = CoGeo<DT>;
-  const int D = ld.D;
   CoTile<MODE, DT, UPG> x{p, tl, ld, lds};
   x.init_fragments(lane);
   const int hf = x.hf, r = 32 * wv + x.n32;
@@ -2656,13 +2643,9 @@ __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoa
   x.st.ok = tok < tl.ntok && x.st.pos >= 0;
   {
     const int qtok = x.st.ok ? tl.q_start + tl.tok0 + tok : tl.q_start;
-    const uint16_t* qp = p.q + ((size_t)qtok * p.Hq + tl.h * p.G + (x.st.ok ? g : 0)) * D;
+    const uint16_t* qp = p.q + ((size_t)qtok * p.Hq + tl.h * p.G + (x.st.ok ? g : 0)) * DT + 8 * hf;
 #pragma unroll
-    for (int s = 0; s < Geo::kSteps; ++s) {  // a narrow row's dims past D are zero
-      const int d = 16 * s + 8 * hf;
-      const u32x4 w = *(const u32x4*)(qp + (d < D ? d : 0));
-      x.q[s] = __builtin_bit_cast(bf16x8, d < D ? w : u32x4{0u, 0u, 0u, 0u});
-    }
+    for (int s = 0; s < Geo::kSteps; ++s) x.q[s] = *(const bf16x8*)(qp + 16 * s);
   }
 #pragma unroll
   for (int d = 0; d < Geo::kDb; ++d) x.st.acc[d] = f32x16{};
@@ -2713,7 +2696,7 @@ __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoa
   // gives the lower half dims 8a .. 8a+7 and the upper half the next eight -- 16-byte stores.  (The
   // swaps need every lane; only the stores are predicated.)
   const float inv = 1.f / lt;
-  uint16_t* op = p.out + ((size_t)(tl.q_start + tl.tok0 + (st.ok ? tok : 0)) * p.Hq + tl.h * p.G + (st.ok ? g : 0)) * D;
+  uint16_t* op = p.out + ((size_t)(tl.q_start + tl.tok0 + (st.ok ? tok : 0)) * p.Hq + tl.h * p.G + (st.ok ? g : 0)) * DT;
 #pragma unroll
   for (int d = 0; d < Geo::kDb; ++d)
 #pragma unroll
@@ -2727,7 +2710,7 @@ __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoa
       const auto s0 = __builtin_amdgcn_permlane32_swap(w[0][0], w[1][0], false, false);
       const auto s1 = __builtin_amdgcn_permlane32_swap(w[0][1], w[1][1], false, false);
       const int dim = 32 * d + 8 * (a + hf);
-      if (st.ok && dim < D)
+      if (st.ok)
         *(u32x4*)(op + dim) = u32x4{(unsigned)s0[0], (unsigned)s1[0], (unsigned)s0[1], (unsigned)s1[1]};
     }
   RPA_TL(ta.write += tl_clock() - tl_c;)
@@ -2818,7 +2801,7 @@ __device__ __forceinline__ int co_tile_parts(int sz, int np) {
 // r / Hkv, kv head r % Hkv.  Calls with more units than kPfOrderMax keep the pair order unsplit.
 template <int MODE, int DT, bool UPG>
 __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], int pf_min, uint8_t* lds, int* s_tile,
-                                        int lane, int wv, int D, int& err, int gpre, bool pf_first) {
+                                        int lane, int wv, int& err, int gpre, bool pf_first) {
   using L = CoLds<MODE, DT, UPG>;
   RPA_TL(tl_set(TL_TILES0, tl_clock());)
   // fixed first positions when every CU holds a prefill-first workgroup (below): b and b + grid/2
@@ -2849,7 +2832,7 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
   int* pkey = (int*)(lds + L::kOrder);
   int* pord = pkey + kPfOrderMax;
   CoLoads<MODE, DT, UPG> ld;
-  ld.init(p, D, wv, lane);
+  ld.init(p, wv, lane);
   __syncthreads();
   if (ranked) {
     for (int u = threadIdx.x; u < nunits; u += blockDim.x) {
@@ -3234,7 +3217,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (pf_total > 0) {
       if (!pf_first) __syncthreads();  // every wave is done with its stream-K LDS regions
       RPA_TL(if (!pf_first) tl_role |= 4;)
-      co_role<MODE, DT, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, D, err, gpre, pf_first);
+      co_role<MODE, DT, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, err, gpre, pf_first);
     }
   }
 
