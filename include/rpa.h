@@ -79,9 +79,11 @@ typedef struct rpa_shape {
  *                  in one 8-wave workgroup per CU; 3 = the tiles in one 8-wave
  *                  workgroup per CU (plain bf16 KV, default mask value, Hkv a
  *                  multiple of 8); 1 = the standalone prefill kernel (page size a
- *                  multiple of 64); 0 = 2, else 1, whichever applies first; -1 =
- *                  causal row blocks of the stream-K role (also whenever none
- *                  applies);
+ *                  multiple of 64); 0 = 2, else 1, whichever applies first (for 64-dim
+ *                  heads, other page sizes than multiples of 32 and Hkv that is no
+ *                  multiple of 4, the kernel weighs the tiles against the row blocks
+ *                  of the batch at hand); -1 = causal row blocks of the stream-K
+ *                  role (also whenever none applies);
  *   prefill_cost   > 0: the cost of one prefill-tile chunk step in stream-K
  *                  units, which sets the work split between the two roles
  *                  (0 = 0.45).

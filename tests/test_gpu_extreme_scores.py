@@ -34,7 +34,7 @@ def test_scores_below_1e30(cuda, path, dim, page):
         for t in range(n - q_lens[i], n):
             want.append(np.repeat(v[: t + 1][at[: t + 1] % 3 == 0].mean(0), 4, axis=0))
     case.kv_pages = kv
-    knobs = dict(prefill_tiles=-1) if path == "rows" else {}
+    knobs = dict(rows=dict(prefill_tiles=-1), tiles=dict(prefill_tiles=2), direct={})[path]
     got = ops.run_case(case, **knobs).float().cpu().numpy()
     want = np.stack(want)
     assert np.all(np.isfinite(got))

@@ -24,7 +24,7 @@ def test_soft_cap_far_above_the_scores(cuda, path, dim, page, dtype, cap):
     lens, q_lens = ([1, 33, 300, 500], [1] * 4) if path == "direct" else ([333, 65, 1200], [70, 65, 16])
     case = make_custom(kv_lens=lens, q_lens=q_lens, num_q_heads=8, num_kv_heads=2, head_dim=dim, page_size=page,
                        pages_per_seq=(512 if path == "direct" else 2048) // page, kv_dtype=dtype, seed=dim + page)
-    knobs = dict(prefill_tiles=-1) if path == "rows" else {}
+    knobs = dict(rows=dict(prefill_tiles=-1), tiles=dict(prefill_tiles=2), direct={})[path]
     got = ops.run_case(case, soft_cap=cap, **knobs).float().cpu().numpy()
     ref = orc.bf16_round(orc.ref_ragged_paged_attention(
         case.q, case.kv_pages, case.kv_lens, case.page_indices, case.cu_q_lens, case.num_seqs, sm_scale=case.sm_scale,

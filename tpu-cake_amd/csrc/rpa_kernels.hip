@@ -199,6 +199,7 @@ struct Params {
   const uint16_t* rel_proj;
   int pf_tq;         // tokens per prefill tile (0 = prefill tiles off)
   int pf_min;        // sequences with at least this many query tokens take prefill tiles
+  int pf_weigh;      // co-resident layout: tiles only where co_worth_tiles finds them ahead
   float pf_cost;     // cost of one prefill tile chunk in stream-K units (work split model)
   // the prefill kernel (rpa_prefill_kernel): when pf_kernel is set, sequences with at least pf_min
   // query tokens are its tiles of pf_tq tokens (256 rows), the attention kernel skips them and
@@ -285,6 +286,19 @@ __device__ __forceinline__ int wave_sum32(int x) {
   x += dpp<0x124, false>(x);  // row_ror:4
   x += dpp<0x128, false>(x);  // row_ror:8: every lane holds its row's total
   return rl(x, 0) + rl(x, 16) + rl(x, 32) + rl(x, 48);
+}
+
+__device__ __forceinline__ int wave_max32(int x) {
+  int y = dpp<0xB1, false>(x);
+  x = x > y ? x : y;
+  y = dpp<0x4E, false>(x);
+  x = x > y ? x : y;
+  y = dpp<0x124, false>(x);
+  x = x > y ? x : y;
+  y = dpp<0x128, false>(x);
+  x = x > y ? x : y;
+  const int a = rl(x, 0) > rl(x, 16) ? rl(x, 0) : rl(x, 16), b = rl(x, 32) > rl(x, 48) ? rl(x, 32) : rl(x, 48);
+  return a > b ? a : b;
 }
 
 __device__ __forceinline__ float wave_sumf(float v) {
@@ -2968,6 +2982,65 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
          tl_set(TL_SETUP, ta.setup); tl_set(TL_LOOP, ta.loop); tl_set(TL_WRITE, ta.write);)
 }
 
+// Whether the batch's sequences of pf_min and more query tokens go to tiles, rather than to stream-K row blocks
+// beside the rest (Params::pf_weigh: the forms other than 128-dim heads at whole-chunk pages and four kv heads per
+// workgroup).  Row blocks spread evenly over the grid but read K and V for every 16 rows, and every wave first
+// walks the longest sequence's blocks; a batch with tiles first ranks and queues them, most after the stream-K
+// ranges, and a tile is at most kCoMaxParts chains of chunk steps.  So, in us:
+//   rows   5 (fp8 at 128 dims: 2) per (16-row block, chunk, head) unit of a wave, 0.25 per block of the longest
+//          sequence
+//   tiles  0.5 (fp8 at 128 dims: 1) per chunk step of the longest chain, 6, and 9 with decode rows in the batch
+// Fitted to 300 random batches (0 to 256 decode rows, 1 to 16 chunks of 16 to 1024 tokens over up to 6000 earlier
+// keys, 64 and 128 dims, 1 to 8 kv heads, pages 16 to 64): the choice itself is 0.2% from the better one in the mean,
+// and weighing costs about 1 us.  Against row blocks for all in the decode layout the batches take 0.72x the time in
+// the mean (one in six 5 to 15% more, mostly 1 to 2 us), with tiles for all 0.81x, but up to 2x: 64 decode rows and
+// one 64-token chunk, fp8, Hq 8 / Hkv 2: 30 us in row blocks, 50 in tiles; 4 chunks of 1024 over 4000 keys: 0.31x in
+// tiles.
+static_assert(kCoMaxParts == 4, "co_worth_tiles' split");
+template <int MODE, int DT>
+__device__ __forceinline__ bool co_worth_tiles(const Params& p, const int kv[4], const int c0[4], const int c1[4],
+                                               int nseq, int lane, int pf_min) {
+  float units = 0.f;
+  int blocks = 0, keys = 0, pairs = 0;
+  bool decode = false;
+#pragma unroll
+  for (int w = 0; w < 4; ++w) {
+    if (nseq <= 64 * w) continue;
+    const int q_len = c1[w] - c0[w], cap = p.PPS * p.S;
+    if (64 * w + lane >= nseq || kv[w] <= 0 || q_len <= 0 || c0[w] < 0 || c1[w] > p.T) continue;
+    if (q_len < pf_min) {
+      decode = true;
+      continue;
+    }
+    const int rb = (q_len * p.G + ROW_BLOCK - 1) / ROW_BLOCK;
+    int last = kv[w] < cap ? kv[w] : cap;
+    float seen = (float)last;  // keys a row block visits, on average; last: the longest tile's
+    if (p.skip_masked) {
+      seen -= 0.5f * (float)q_len;
+      if (p.sliding_window > 0) {
+        seen = fminf(seen, (float)p.sliding_window);
+        last = last - p.pf_tq < p.sliding_window ? last : p.sliding_window + p.pf_tq;
+      }
+    }
+    units += (float)rb * (seen * (1.f / KV_CHUNK) + 0.5f);
+    blocks = rb > blocks ? rb : blocks;
+    keys = last > keys ? last : keys;
+    pairs += (rb + 7) >> 3;  // (tiles of 128 rows)
+  }
+  if (__ballot(pairs > 0) == 0) return true;
+  units = wave_sumf(units) * (float)p.Hkv * __builtin_amdgcn_rcpf((float)(p.grid * kCoWaves));
+  blocks = wave_max32(blocks);
+  keys = wave_max32(keys);
+  const int tiles = wave_sum32(pairs) * p.Hkv;
+  float steps = (float)((keys + KV_CHUNK - 1) / KV_CHUNK);
+  if (tiles <= p.co_split_max)  // (as co_role splits them)
+    steps *= 4 * tiles <= p.grid ? 0.25f : 3 * tiles <= p.grid ? 0.33f : 2 * tiles <= p.grid ? 0.5f : 1.f;
+  constexpr bool kWideFp8 = MODE == KV_FP8 && DT == kD;
+  const float rows_us = (kWideFp8 ? 2.f : 5.f) * units + 0.25f * (float)blocks;
+  const float tiles_us = (kWideFp8 ? 1.f : 0.5f) * steps + (__ballot(decode) != 0 ? 15.f : 6.f);
+  return rows_us > tiles_us;
+}
+
 // CO: the co-resident layout's instantiation (p.co set), with the co-resident prefill role; the
 // other instantiations carry the 8-wave prefill role (plain bf16 KV) or none, so the decode-only
 // launches keep the registers of a kernel without the co-resident role.
@@ -3031,6 +3104,8 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (fz) tv = nseq;
     // prefill tiles need the whole metadata in the four windows
     pf_min = (kTiles && p.pf_tq > 0 && nseq <= 64 * kWin) ? p.pf_min : 0;
+    if constexpr (CO)
+      if (p.pf_weigh && pf_min > 0 && !co_worth_tiles<MODE, DT>(p, kv, c0, c1, nseq, lane, pf_min)) pf_min = 0;
 #pragma unroll
     for (int w = 0; w < kWin; ++w) {
       wsi[w] = SeqInfo{0, 0, 0, 0};
@@ -5322,10 +5397,14 @@ int nominal_per_cu(int hg, size_t lds) {
 //       128-dim heads, bf16 KV (plain or with scalar k/v scales) or fp8 KV, page size a multiple of 32, Hkv
 //       a multiple of 4: a workgroup is one stream-K worker of four kv heads;
 //       128- or 64-dim heads, plain bf16 or fp8 KV, any other page size or kv head count: a workgroup holds
-//       4 / HG workers -- except where the 8-wave layout below takes plain bf16 pools.  As 16-row stream-K
-//       blocks those rows read K and V again for every 16 of them: a page-16 chunked prefill (5 chunks of up
-//       to 1023 tokens, Hq 8 / Hkv 2) took 145 us a call against 59 in tiles, a 64-dim mixed batch (24
-//       decode rows, 4 chunks of 512, Hq 32 / Hkv 8) 353 against 78;
+//       4 / HG workers, and with prefill_tiles 0 the kernel weighs tiles against row blocks (co_worth_tiles)
+//       -- except where the 8-wave layout below takes plain bf16 pools.  As 16-row stream-K blocks those rows
+//       read K and V again for every 16 of them: a page-16 chunked prefill (5 chunks of up to 1023 tokens,
+//       Hq 8 / Hkv 2) took 145 us a call against 59 in tiles, a 64-dim mixed batch (24 decode rows, 4 chunks
+//       of 512, Hq 32 / Hkv 8) 353 against 78.  (The exception is kept from before the tiles took such pages,
+//       and is a trade: 4 prompts of 2048, page 16, Hq 32 / Hkv 8, 252 us in the 8-wave layout, 200 in this one,
+//       page 24 254 / 198, 24 decode rows beside 4 chunks of 512 211 / 158; but beside one chunk of 64 95 / 97, and
+//       with Hq 16 / Hkv 16 183 / 212 and 154 / 167);
 //   prefill_tiles 3, or 2 / 0 otherwise, for plain bf16 KV whose masked keys get weight 0 and
 //     eight kv heads per workgroup: the attention kernel's tiles in 8-wave workgroups, one per
 //     CU, roles split by CU;
@@ -5357,6 +5436,7 @@ void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_opt
     p.lockstep = p.HG == kCoWaves;
     p.pf_tq = 32 * kCoWaves / p.G;
     p.pf_min = 16;
+    p.pf_weigh = !co_one && pt == 0;
     p.pf_cost = cost;
   } else if (pk_ok && (pt == 1 || (pt == 0 && !tiles_ok))) {
     p.pf_kernel = true;
@@ -5502,7 +5582,10 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   // slots of 128 rows over its partial areas (2 x 256 rows per CU)
   static_assert(kCoMaxParts * 128 <= 2 * kPkRows, "co split tiles exceed the prefill-kernel partial areas");
   if (p.co) {
-    p.co_split_max = d.cus;
+    // at most the tiles the batch can hold (the combine launch has four workgroups for each)
+    const long long seqs = shape->num_tokens / p.pf_min < p.Nmax ? shape->num_tokens / p.pf_min : p.Nmax;
+    const long long tiles = (shape->num_tokens / p.pf_tq + seqs) * p.Hkv;
+    p.co_split_max = tiles < d.cus ? (int)tiles : d.cus;
     p.co_desc = (CoDesc*)((uint8_t*)workspace + w.co_desc);
   }
   if (ev_begin && hipEventRecord((hipEvent_t)ev_begin, st) != hipSuccess)
