@@ -1248,7 +1248,12 @@ __device__ __forceinline__ void step(const Params& p, int nseq, int lane, int n,
 // row in the lane that looked the key's page up (line_addr).  Pages of 16, against the operand
 // layout above, 64 sequences of ~2048 keys, 8 kv heads: 128-dim heads 121 -> 107 us, 64-dim 106 ->
 // 59 (rows of 64 elements fixed at compile time), 256-dim (4 kv heads) 132 -> 108, a window of 512
-// 42 -> 37.  fp8 has its own layout, and the v1 bias there is added in the operand layout.
+// 42 -> 37.  Not where more than 16 query heads share a kv head, 128-dim heads or wider than 64 with at most
+// two kv heads (operand_rows): the row blocks after a key's first find its rows in cache, and the tile's extra
+// steps then cost more than the half lines; pages of 16, operand layout / whole rows: 1 kv head, G 32, 128 dims,
+// 48 sequences of up to 3000 keys 36.8 / 41.4 us, 128 of up to 6000 83.8 / 90.4, 112 dims 85.9 / 98.6; 4 kv heads
+// 286 / 299; but 64 dims 71.6 / 58.2, 256 dims and 3 kv heads 553 / 398.  fp8 has its own layout, and the v1 bias
+// there is added in the operand layout.
 template <int MODE, bool UPG>
 struct LinePath {
   static constexpr bool on = MODE == KV_BF16 || MODE == KV_BF16_SCALED || MODE == KV_BF16_FUSED ||
@@ -3048,7 +3053,8 @@ __device__ __forceinline__ bool co_worth_tiles(const Params& p, const int kv[4],
 // only, every row through stream-K).  DN: a narrow
 // head dim of 32 or 64 fixed at compile time, whose full-line loads read whole DN-element rows
 // (Lines<DN>).
-template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0>
+// OPL: the decode role in the operand layout where the full-line path exists (operand_rows).
+template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0, bool OPL = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rpa_attn_kernel(Params p) {
   static_assert(DN == 0 || (NW && (DN == 64 || (UPG && DN == 32))), "DN: a narrow instantiation of 32 or 64");
   static_assert(!CO || co_tiles<MODE>(), "CO: a mode with co-resident tiles");
@@ -3234,7 +3240,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
         advance<MODE>(p, nseq, lane, win, nxt, err);
       else
         nxt.nch = 0;
-      constexpr bool kLine = LinePath<MODE, UPG>::on;
+      constexpr bool kLine = LinePath<MODE, UPG>::on && !OPL;
       const Pages pg_cur = load_pages<MODE, UPG, kLine>(p, cur, n);
       Pages pg_nxt = load_pages<MODE, UPG, kLine>(p, nxt, n);
       if constexpr (kLine) {
@@ -5449,6 +5455,12 @@ void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_opt
   }
 }
 
+// Whether decode rows keep the operand layout where the full-line path exists (LinePath, with both sides).
+bool operand_rows(const Params& p, int mode) {
+  return (mode == KV_BF16 || mode == KV_BF16_SCALED) && p.S % KV_CHUNK != 0 && !p.co && p.G > ROW_BLOCK &&
+         (p.D == kD || (p.D > 64 && p.Hkv <= 2));
+}
+
 // LDS of a co-resident workgroup's tile role.
 size_t co_lds_bytes(int mode, bool upg, int D) {
   const bool fp8 = mode == KV_FP8;
@@ -5591,6 +5603,7 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   if (ev_begin && hipEventRecord((hipEvent_t)ev_begin, st) != hipSuccess)
     return fail(RPA_E_HIP, "hipEventRecord(begin) failed");
   const bool upg = p.S % KV_CHUNK == 0;
+  const bool opl = operand_rows(p, mode);
   const dim3 grid(p.grid), block(64 * waves);
   size_t lds = (size_t)p.HG * (kVtBytes + (mode == KV_BF16_FUSED ? kRelStage : 0) + (p.D > kD ? kWideSlot : 0));
   if (p.co) {
@@ -5622,12 +5635,14 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
       else if (upg && p.D == 32) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, false, true, 32>), grid, block, lds, st, p);
       else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, false, true>), grid, block, lds, st, p);
       else if (p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, true, 64>), grid, block, lds, st, p);
+      else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, true, 0, 0, true>), grid, block, lds, st, p);
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, true>), grid, block, lds, st, p);
     } else {
       if (upg && p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true, 64>), grid, block, lds, st, p);
       else if (upg && p.D == 32) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true, 32>), grid, block, lds, st, p);
       else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, false, true>), grid, block, lds, st, p);
       else if (p.D == 64) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true, 64>), grid, block, lds, st, p);
+      else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true, 0, 0, true>), grid, block, lds, st, p);
       else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, true>), grid, block, lds, st, p);
     }
   } else if (mode == KV_FP8) {
@@ -5638,11 +5653,13 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
   } else if (mode == KV_BF16_SCALED) {
     if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true, true>), grid, block, lds, st, p);
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, true>), grid, block, lds, st, p);
+    else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, false, 0, 0, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false>), grid, block, lds, st, p);
   } else {
     if (p.co && upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true>), grid, block, lds, st, p);
     else if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true>), grid, block, lds, st, p);
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true>), grid, block, lds, st, p);
+    else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, false, 0, 0, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false>), grid, block, lds, st, p);
   }
   hipError_t e = hipGetLastError();
