@@ -243,7 +243,10 @@ int rpa_timeline_read(int64_t* host_rows, int32_t rows, void* stream);
  * With head_dim a multiple of 8 in [32, 128], 16-byte aligned tensors, P * S < 2^31 and R in
  * {0, 16} with E a multiple of 8 -- any page size -- the step is one attention launch (new token
  * read from keys/values, bias formed in the kernel) plus the merge launch, which also stores the
- * token; other shapes take a preparation launch first (cache write, page table, bias table).
+ * token, or for small calls (as rpa_options_t says of the operator's) one launch in all; other
+ * shapes take a preparation launch first (cache write, page table, bias table).  The page a token
+ * is written to belongs to its sequence alone (the preflight rejects a shared one): in one launch
+ * the store and other sequences' reads are not ordered.
  * --------------------------------------------------------------------------------------- */
 typedef struct rpa_fused_shape {
   int32_t num_seqs;          /* B */
@@ -284,10 +287,13 @@ int rpa_inkling_fused_decode(const rpa_fused_shape_t* shape, float sm_scale, con
  * over the keys l < sequence_lengths[b] of pages page_table[b, :]; the oracle's scale is 1/D.
  * Separate key and value caches; bias indexed by key position (bias_len >= every length).
  * The reference's `experiment inkling-rpa` renders the experiment artifact for this workload
- * (cli.py:667-676); this entry executes it.  The caches are packed into the operator's
- * combined layout in the workspace on every call (a copy of the whole cache: this entry serves
- * the contract's shapes; a serving cache belongs in the combined layout of
- * rpa_ragged_paged_attention).
+ * (cli.py:667-676); this entry executes it.  Short page tables (up to 4096 keys, fewer with
+ * few sequences over a small cache; head_dim a multiple of 8; query and caches 16-byte and out
+ * 8-byte aligned) take one launch over the caches in place.  Other calls pack the caches into
+ * the operator's combined layout in the workspace every time (a copy of the whole cache: this
+ * entry serves the contract's shapes; a serving cache belongs in the combined layout of
+ * rpa_ragged_paged_attention); the workspace size covers either form.  out may alias query
+ * below 128 dims only.
  * --------------------------------------------------------------------------------------- */
 typedef struct rpa_inkling_shape {
   int32_t num_seqs;       /* B */

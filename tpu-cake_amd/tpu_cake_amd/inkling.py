@@ -5,8 +5,9 @@
 sequence, separate key and value caches ``[P, S, Hkv, D]``, a ``[B, MP]`` page table, a bias
 ``[H, L]`` indexed by key position, scale ``1/D``; it returns ``[B, H, D]``.  The reference renders
 this workload's experiment artifact (``src/tpu_cake/cli.py:667-676``, contract
-``inkling_rpa.py:693-723``); here it runs through the C ABI entry ``rpa_inkling_decode`` (the
-operator's kernels in relative-bias mode after one packing launch).
+``inkling_rpa.py:693-723``); here it runs through the C ABI entry ``rpa_inkling_decode``: one
+launch over the caches in place for short page tables, else the operator's kernels in
+relative-bias mode after one packing launch.
 
 Inputs are torch tensors on the GPU: bf16 query, caches and bias (the contract's dtypes), int32
 page table and lengths.  Key and value caches must have the same heads and head dim (the
