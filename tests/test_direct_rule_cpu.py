@@ -50,8 +50,8 @@ def test_schedule_knobs_keep_their_launches(dtype, knobs, direct):
     (dict(slots=4, tokens=4, hkv=1, g=32), False), (dict(slots=4, tokens=4, hkv=1, g=32, keys=512), True),
     (dict(slots=14, tokens=14, hkv=1, g=32), True), (dict(slots=4, tokens=4, hkv=1, g=64, keys=256), False),
     (dict(slots=4, tokens=4, hkv=1, g=64, keys=128), True), (dict(hkv=1, g=64, keys=512), True),
-    (dict(hkv=1, g=65, keys=64), False), (dict(slots=128, g=32, keys=192), False),
-    (dict(slots=128, g=32, keys=128), True)])
+    (dict(hkv=1, g=65, keys=64), False), (dict(slots=128, g=32, keys=576), False),
+    (dict(slots=128, g=32, keys=512), True), (dict(slots=65, g=64, keys=256), True)])
 def test_bounds(kw, direct):
     case = _case(**kw)
     assert _direct(case) == direct

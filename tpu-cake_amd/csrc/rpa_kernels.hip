@@ -4181,6 +4181,7 @@ struct DirectArgs {
   const uint16_t* bias;  // v1: [Hq, bias_len] by key position
   int bias_len;
   uint32_t pmagic;       // ceil(2^31 / S): page_of below 4096 keys is one multiplication
+  int tpb;               // tokens of a block of query rows: 16 / G, at least 1
 };
 
 // K or V of a chunk as it comes from memory, whole rows per load: load i covers keys kKeys i ..
@@ -4292,7 +4293,6 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   }
   if (live && ql > kv) err |= ERR_QLEN;
   int tok = 0;  // the block's first token in its sequence
-  const int tpb = p.G < ROW_BLOCK ? ROW_BLOCK / p.G : 1;  // tokens of a block
   if constexpr (!kFused && !kV1) {
     // the block that starts at token `slot`, if one does.  One token per sequence: sequence `slot`'s, whose
     // metadata is here; otherwise the token's sequence is looked up
@@ -4313,7 +4313,7 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
           }
         }
       }
-      live = live && (slot - q0) % tpb == 0;
+      live = live && (slot - q0) % a.tpb == 0;
       if (live) {
         kv = uni(p.kv_lens[i]);
         kv = kv > cap ? (int)cap : (kv < 0 ? 0 : kv);
@@ -4323,7 +4323,7 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
       }
     }
     tok = slot - q0;
-    live = live && tok % tpb == 0;
+    if (tok != 0) live = live && tok % a.tpb == 0;
   }
   if constexpr (kFused) {  // (make_fused_seq) the sequence's pages start at entry cu_kv / S
     const int cu = uni(c1), pb = page_of(cu, p), npg = kv > 0 ? page(kv - 1) + 1 : 0;
@@ -4339,7 +4339,7 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
   live = live && ql > 0 && kv > 0;
 
   // the block's tokens q0 .. q0 + ntok - 1, at key positions pos0 .., and the chunks its rows see
-  const int ntok = kFused || kV1 ? 1 : ql - tok < tpb ? ql - tok : tpb, rows = live ? ntok * p.G : 0;
+  const int ntok = kFused || kV1 ? 1 : ql - tok < a.tpb ? ql - tok : a.tpb, rows = live ? ntok * p.G : 0;
   const int pos0 = kv - ql + tok;
   q0 += tok;
   const int vis = p.skip_masked && pos0 + ntok < kv ? pos0 + ntok : kv;
@@ -4648,8 +4648,8 @@ __global__ void rpa_attn_kernel_direct(Params p, DirectArgs a) {
 //   G 17 to 64, t = 2 to 4 turns: to 2^(1-t) of the elements, which few pairs do not lose (4 pairs: G 32, 512 keys
 //     19.6 / 15.1, 1024 keys 23.3 / 21.3, 14.3 / 21.9; G 48, 256 keys 17.2 / 15.1; G 64, 128 keys 16.3 / 15.0, 512
 //     keys 20.3 / 27.5), to 3 / t of them from 7 t pairs on (G 32, 14 pairs of 1024 keys 24.2 / 19.8, 20.1 / 22.4;
-//     G 48, 24 pairs 31.4 / 28.1; G 64, 48 pairs of 512 keys 30.0 / 28.6, 40.1 / 29.0); a second round to 1 / 4 t
-//     (G 32, 512 pairs of 128 keys 41.7 / 18.2).
+//     G 48, 24 pairs 31.4 / 28.1; G 64, 48 pairs of 512 keys 30.0 / 28.6, 40.1 / 29.0); a second round to 1 / t
+//     (512 pairs: G 24, 512 keys 53.9 / 38.4, 76.1 / 56.3; G 64, 256 keys 63.3 / 45.5, 66.3 / 52.4).
 //   G > 64: never (G 128, 64 keys 17.3 / 22.4; 1024 keys 30.1 / 76.9).
 bool direct_fits(long long cap, int D, bool fp8, int G, long long pairs) {
   const long long elems = cap * (D < 64 ? 64 : D);
@@ -4658,7 +4658,7 @@ bool direct_fits(long long cap, int D, bool fp8, int G, long long pairs) {
   if (pairs > kDirectPairs) {
     const bool wide = D > 64 && D <= 128;
     const int share = fp8 ? (wide ? 4 : 1) : D < 64 ? 1 : D <= 128 ? 2 : 8;
-    return elems <= kDirectElems / share && (turns == 1 || elems * turns <= kDirectElems / 4);
+    return turns == 1 ? elems <= kDirectElems / share : elems * turns <= kDirectElems;
   }
   return turns == 1 || elems << (turns - 1) <= kDirectElems ||
          (pairs >= 7 * turns && elems * turns <= 3 * kDirectElems);
@@ -4695,6 +4695,7 @@ bool direct_call(const rpa_shape_t* s, const rpa_options_t* o) {
 template <int MODE, int DW>
 void launch_direct_kernel(const Params& p, DirectArgs a, hipStream_t st) {
   a.pmagic = (uint32_t)(((1ull << 31) + p.S - 1) / p.S);
+  a.tpb = p.G < ROW_BLOCK ? ROW_BLOCK / p.G : 1;
   constexpr size_t lds = kDirectWaves * (KV_CHUNK * (2 * DW + 32) + 16 * 2 * sizeof(float));
   hipLaunchKernelGGL((rpa_attn_kernel_direct<MODE, DW>), dim3(p.Nmax * p.Hkv), dim3(64 * kDirectWaves), lds, st, p, a);
 }

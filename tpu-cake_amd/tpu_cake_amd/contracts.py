@@ -358,7 +358,7 @@ def direct_call(num_tokens: int, max_num_seqs: int, hkv: int, head_dim: int, tab
             share = 4 if 64 < head_dim <= 128 else 1
         else:
             share = 1 if head_dim < 64 else 2 if head_dim <= 128 else 8
-        return elems <= DIRECT_ELEMS // share and (turns == 1 or elems * turns <= DIRECT_ELEMS // 4)
+        return elems <= DIRECT_ELEMS // share if turns == 1 else elems * turns <= DIRECT_ELEMS
     return (turns == 1 or elems << (turns - 1) <= DIRECT_ELEMS
             or (pairs >= 7 * turns and elems * turns <= 3 * DIRECT_ELEMS))
 
