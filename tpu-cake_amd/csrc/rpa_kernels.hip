@@ -1699,10 +1699,6 @@ __device__ __forceinline__ bf16x8 pf_softmax_plain_m(const Params& p, const f32x
   return __builtin_bit_cast(bf16x8, pw);
 }
 
-__device__ __forceinline__ bf16x8 pf_softmax_plain(const Params& p, const f32x4 sc[2], PfRow& st) {
-  return pf_softmax_plain_m(p, sc, st, rows4_max(pf_lane_max(sc)));
-}
-
 // One chunk for one 16-row block: scores sc[kb] (keys 16kb + 4j + rr of row n), softmax update,
 // P^T packed for the PV MFMA.
 __device__ __forceinline__ bf16x8 pf_softmax(const Params& p, const PfTile& tl, int c, const f32x4 sc[2], PfRow& st,
@@ -5405,6 +5401,7 @@ int nominal_per_cu(int hg, size_t lds) {
 //       a multiple of 4: a workgroup is one stream-K worker of four kv heads;
 //       128- or 64-dim heads, plain bf16 or fp8 KV, any other page size or kv head count: a workgroup holds
 //       4 / HG workers, and with prefill_tiles 0 the kernel weighs tiles against row blocks (co_worth_tiles)
+//       (scalar scales there have no tile instantiation: row blocks, as ever)
 //       -- except where the 8-wave layout below takes plain bf16 pools.  As 16-row stream-K blocks those rows
 //       read K and V again for every 16 of them: a page-16 chunked prefill (5 chunks of up to 1023 tokens,
 //       Hq 8 / Hkv 2) took 145 us a call against 59 in tiles, a 64-dim mixed batch (24 decode rows, 4 chunks
