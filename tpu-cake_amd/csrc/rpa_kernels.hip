@@ -67,6 +67,7 @@ constexpr int kWaveLds = kVtBytes_ + kKtBytes;  // LDS per decode wave: V region
 constexpr int kMaxWavesPerCU = 8;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kRescaleLog2 = 8.f;  // lazy softmax rescale threshold (log2 units)
+constexpr float kDirectNegligible = 24.f; // log2: below it, a chunk's probabilities are lost beside the others' in fp32
 constexpr float kDefaultMask = -0.7f * 3.4028234663852886e38f;  // ragged_paged_attention.py:32
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -200,6 +201,7 @@ struct Params {
   int pf_tq;         // tokens per prefill tile (0 = prefill tiles off)
   int pf_min;        // sequences with at least this many query tokens take prefill tiles
   int pf_weigh;      // co-resident layout: tiles only where co_worth_tiles finds them ahead
+  int pf_exact;      // co-resident layout: CoTile's EX
   float pf_cost;     // cost of one prefill tile chunk in stream-K units (work split model)
   // the prefill kernel (rpa_prefill_kernel): when pf_kernel is set, sequences with at least pf_min
   // query tokens are its tiles of pf_tq tokens (256 rows), the attention kernel skips them and
@@ -2234,7 +2236,12 @@ __device__ __forceinline__ float halves_sum(float v) {
 }
 
 // The tile's chunk stream and compute.  All members are wave-uniform or per-lane registers.
-template <int MODE, int DT, bool UPG>
+// EX: an instantiation that can move the reference with every chunk (`exact`), by the least that makes its largest
+// probability a power of two, as the one-launch kernel does, instead of lazily.  For batches that the prefill kernel
+// would cut into short chains over all CUs, whose error the lazily moved maximum of a longer chain does not reach:
+// two prompts of 943 and 475 tokens, one kv head, page 64, relative error against float64 0.002225 there, 0.002322
+// lazily, 0.002019 exact (48.8, 39.2 and 41 us).
+template <int MODE, int DT, bool UPG, bool EX>
 struct CoTile {
   using L = CoLds<MODE, DT, UPG>;
   using Geo = CoGeo<DT>;
@@ -2249,6 +2256,7 @@ struct CoTile {
   bf16x8 ka[Geo::kSteps];          // the A fragments of K of chunk c + 1 at the start of step c
   const uint8_t* vb[3];            // UPG: addresses (base_of) of chunks c + 2 .. c + 4 (fp8 one further)
   u32x2 ent;                       // UPG: the table entry of the chunk whose K step c issues
+  bool exact;                      // EX: see above
   int c_tail;                      // the chunk with keys past kv_len (-1: none)
   int plain_to;                    // chunks below it need no masking
   typedef __attribute__((address_space(3))) const uint8_t* lds_cp;
@@ -2439,8 +2447,14 @@ struct CoTile {
       } else if (it == 2) {
         ma = halves_max(fmaxf(ma, mb));
         const float mc = PLAIN ? ma * sl2 : ma;
-        grow = mc > st.m + kRescaleLog2;
-        mn = grow ? mc : st.m;
+        if constexpr (EX) {
+          const float up = mc - st.m;
+          grow = mc > st.m + (exact ? -kDirectNegligible : kRescaleLog2);
+          mn = !grow ? st.m : up > kRescaleLog2 ? mc : mc - rintf(up);
+        } else {
+          grow = mc > st.m + kRescaleLog2;
+          mn = grow ? mc : st.m;
+        }
       } else if (it < 19) {
         const int i = it - 3;
         e[i] = __builtin_amdgcn_exp2f(PLAIN ? __builtin_fmaf(s[i], sl2, -mn) : x[i] - mn);
@@ -2645,12 +2659,13 @@ struct CoTile {
 };
 
 // slot >= 0: the tile is one part of a split tile, its (m, l, acc) go to that partial slot
-template <int MODE, int DT, bool UPG>
+template <int MODE, int DT, bool UPG, bool EX>
 __device__ __forceinline__ void co_tile(const Params& p, const PfTile& tl, CoLoads<MODE, DT, UPG>& ld,
-                                        uint8_t* lds, int wv, int lane, int& err, int slot, TlAcc& ta) {
+                                        uint8_t* lds, int wv, int lane, int& err, int slot, bool exact, TlAcc& ta) {
   using L = CoLds<MODE, DT, UPG>;
   using Geo = CoGeo<DT>;
-  CoTile<MODE, DT, UPG> x{p, tl, ld, lds};
+  CoTile<MODE, DT, UPG, EX> x{p, tl, ld, lds};
+  x.exact = exact;
   x.init_fragments(lane);
   const int hf = x.hf, r = 32 * wv + x.n32;
   const int tok = r / p.G, g = r - tok * p.G;
@@ -2814,9 +2829,9 @@ __device__ __forceinline__ int co_tile_parts(int sz, int np) {
 // workgroup writes every unit's key (one thread per unit: a binary search over the sequences'
 // first pairs finds its sequence), ranks them in LDS and maps queue position r to the unit of rank
 // r / Hkv, kv head r % Hkv.  Calls with more units than kPfOrderMax keep the pair order unsplit.
-template <int MODE, int DT, bool UPG>
+template <int MODE, int DT, bool UPG, bool EX>
 __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], int pf_min, uint8_t* lds, int* s_tile,
-                                        int lane, int wv, int& err, int gpre, bool pf_first) {
+                                        int lane, int wv, int& err, int gpre, bool pf_first, bool exact) {
   using L = CoLds<MODE, DT, UPG>;
   RPA_TL(tl_set(TL_TILES0, tl_clock());)
   // fixed first positions when every CU holds a prefill-first workgroup (below): b and b + grid/2
@@ -2977,7 +2992,7 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
         d->valid[threadIdx.x] = 1;
       }
     }
-    co_tile<MODE, DT, UPG>(p, tl, ld, lds, wv, lane, err, slot, ta);
+    co_tile<MODE, DT, UPG, EX>(p, tl, ld, lds, wv, lane, err, slot, exact, ta);
   }
   RPA_TL(tl_set(TL_NTILES, ta.tiles); tl_set(TL_NSTEPS, ta.steps); tl_set(TL_QUEUE, ta.queue);
          tl_set(TL_SETUP, ta.setup); tl_set(TL_LOOP, ta.loop); tl_set(TL_WRITE, ta.write);)
@@ -2997,10 +3012,13 @@ __device__ __forceinline__ void co_role(const Params& p, const SeqInfo wsi[4], i
 // the mean (one in six 5 to 15% more, mostly 1 to 2 us), with tiles for all 0.81x, but up to 2x: 64 decode rows and
 // one 64-token chunk, fp8, Hq 8 / Hkv 2: 30 us in row blocks, 50 in tiles; 4 chunks of 1024 over 4000 keys: 0.31x in
 // tiles.
+// exact: whether CoTile's EX moves the reference with every chunk: up to 8 of the prefill kernel's 64-key steps of 256
+// rows per CU (a wave's unit here is 1 / 32 of one, and eight waves share a CU).
+constexpr float kCoExactUnits = 32.f;
 static_assert(kCoMaxParts == 4, "co_worth_tiles' split");
 template <int MODE, int DT>
 __device__ __forceinline__ bool co_worth_tiles(const Params& p, const int kv[4], const int c0[4], const int c1[4],
-                                               int nseq, int lane, int pf_min) {
+                                               int nseq, int lane, int pf_min, bool& exact) {
   float units = 0.f;
   int blocks = 0, keys = 0, pairs = 0;
   bool decode = false;
@@ -3030,6 +3048,7 @@ __device__ __forceinline__ bool co_worth_tiles(const Params& p, const int kv[4],
   }
   if (__ballot(pairs > 0) == 0) return true;
   units = wave_sumf(units) * (float)p.Hkv * __builtin_amdgcn_rcpf((float)(p.grid * kCoWaves));
+  exact = units < kCoExactUnits;
   blocks = wave_max32(blocks);
   keys = wave_max32(keys);
   const int tiles = wave_sum32(pairs) * p.Hkv;
@@ -3050,7 +3069,8 @@ __device__ __forceinline__ bool co_worth_tiles(const Params& p, const int kv[4],
 // head dim of 32 or 64 fixed at compile time, whose full-line loads read whole DN-element rows
 // (Lines<DN>).
 // OPL: the decode role in the operand layout where the full-line path exists (operand_rows).
-template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0, bool OPL = false>
+template <int MODE, bool UPG, bool CO = false, bool NW = false, int DN = 0, int DT = CO ? kD : 0, bool OPL = false,
+          bool EX = false>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) void rpa_attn_kernel(Params p) {
   static_assert(DN == 0 || (NW && (DN == 64 || (UPG && DN == 32))), "DN: a narrow instantiation of 32 or 64");
   static_assert(!CO || co_tiles<MODE>(), "CO: a mode with co-resident tiles");
@@ -3075,6 +3095,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
   Window win;
   SeqInfo wsi[kWin];
   int nseq, tv, pf_min;
+  bool exact = true;  // (co_worth_tiles)
   {
     int kv[kWin], c0[kWin], c1[kWin];
     // fused decode step: q rows 0..B-1 one per sequence, cu_kv in place of the second q bound
@@ -3107,7 +3128,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     // prefill tiles need the whole metadata in the four windows
     pf_min = (kTiles && p.pf_tq > 0 && nseq <= 64 * kWin) ? p.pf_min : 0;
     if constexpr (CO)
-      if (p.pf_weigh && pf_min > 0 && !co_worth_tiles<MODE, DT>(p, kv, c0, c1, nseq, lane, pf_min)) pf_min = 0;
+      if (p.pf_weigh && pf_min > 0 && !co_worth_tiles<MODE, DT>(p, kv, c0, c1, nseq, lane, pf_min, exact)) pf_min = 0;
 #pragma unroll
     for (int w = 0; w < kWin; ++w) {
       wsi[w] = SeqInfo{0, 0, 0, 0};
@@ -3294,7 +3315,7 @@ __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2))) voi
     if (pf_total > 0) {
       if (!pf_first) __syncthreads();  // every wave is done with its stream-K LDS regions
       RPA_TL(if (!pf_first) tl_role |= 4;)
-      co_role<MODE, DT, UPG>(p, wsi, pf_min, smem, &s_tile, lane, wv, err, gpre, pf_first);
+      co_role<MODE, DT, UPG, EX>(p, wsi, pf_min, smem, &s_tile, lane, wv, err, gpre, pf_first, exact);
     }
   }
 
@@ -4166,7 +4187,6 @@ __global__ __launch_bounds__(64 * CW) __attribute__((amdgpu_waves_per_eu(4))) vo
 constexpr int kDirectWaves = 8;
 constexpr int kDirectElems = 1024 * 128;  // keys of a page table x row width
 constexpr int kDirectPairs = 256;         // (sequence slot, kv head) pairs of one round: a workgroup fills a CU
-constexpr float kDirectNegligible = 24.f; // log2: below it, a chunk's probabilities are lost beside the others' in fp32
 constexpr int kDirectMaxKeys = 4096;      // (pmagic's range)
 
 struct DirectArgs {
@@ -5441,6 +5461,7 @@ void resolve_layout(Params& p, int mode, const rpa_shape_t* shape, const rpa_opt
     p.pf_tq = 32 * kCoWaves / p.G;
     p.pf_min = 16;
     p.pf_weigh = !co_one && pt == 0;
+    p.pf_exact = !co_one;
     p.pf_cost = cost;
   } else if (pk_ok && (pt == 1 || (pt == 0 && !tiles_ok))) {
     p.pf_kernel = true;
@@ -5654,7 +5675,8 @@ static int launch_rpa(const rpa_shape_t* shape, const rpa_options_t* opt, const 
     else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false, false, false, 0, 0, true>), grid, block, lds, st, p);
     else hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16_SCALED, false>), grid, block, lds, st, p);
   } else {
-    if (p.co && upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true>), grid, block, lds, st, p);
+    if (p.co && upg && p.pf_exact) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true, false, 0, kD, false, true>), grid, block, lds, st, p);
+    else if (p.co && upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true, true>), grid, block, lds, st, p);
     else if (p.co) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, true>), grid, block, lds, st, p);
     else if (upg) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, true>), grid, block, lds, st, p);
     else if (opl) hipLaunchKernelGGL((rpa_attn_kernel<KV_BF16, false, false, false, 0, 0, true>), grid, block, lds, st, p);
