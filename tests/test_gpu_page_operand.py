@@ -32,3 +32,17 @@ def test_groups_past_16(cuda, dim, page, hkv, g, kw):
     assert np.all(np.isfinite(got))
     assert np.allclose(got, ref, atol=0.02, rtol=0.02)
     assert np.max(np.abs(got - ref)[np.abs(ref) < 4], initial=0.0) <= 2e-2
+
+
+@pytest.mark.parametrize("hkv,g,tiles", [(8, 20, 3), (8, 17, 0), (2, 32, -1)])
+def test_groups_past_16_beside_a_prompt(cuda, hkv, g, tiles):
+    print(f"[case] Hkv {hkv} G {g} prefill_tiles {tiles}", flush=True)
+    case = make_custom(kv_lens=[700, 33, 150], q_lens=[1, 1, 70], num_q_heads=hkv * g, num_kv_heads=hkv, page_size=16,
+                       seed=hkv + g)
+    got = ops.run_case(case, prefill_tiles=tiles).float().cpu().numpy()
+    ref = orc.bf16_round(orc.ref_ragged_paged_attention(
+        case.q, case.kv_pages, case.kv_lens, case.page_indices, case.cu_q_lens, case.num_seqs, sm_scale=case.sm_scale,
+        probs_bf16=True))
+    assert np.all(np.isfinite(got))
+    assert np.allclose(got, ref, atol=0.02, rtol=0.02)
+    assert np.max(np.abs(got - ref)[np.abs(ref) < 4], initial=0.0) <= 2e-2
